@@ -892,11 +892,16 @@ __global__ __launch_bounds__(64 * NW, WPE) void bwd_rows2_kernel(BwdParams prm) 
 // ---------------------------------------------------------------------------
 // Cols kernel.
 // ---------------------------------------------------------------------------
-template <int HP, int D, int C, int RC>
+// NW waves of 64 lanes per workgroup, each head-owner of HP / NW heads; OCC
+// waves per SIMD (4 OCC / NW workgroups per CU). Four waves are row-owners of
+// RC / 16 row groups of four rows each, eight of half a row group (two rows).
+template <int HP, int D, int C, int RC, int NW = 4, int OCC = 2>
 struct Cols2Cfg {
-  static constexpr int HW = HP / 4, NS = RC / 16, NCT = C / 16;
+  static constexpr int HW = HP / NW, NS = RC / 16, NCT = C / 16;
   static constexpr int RG = RC / 4;     // row groups per chunk
-  static constexpr int RGW = RC / 16;   // row groups per row-owner wave
+  static constexpr int RGW = RC / 16;   // row groups per row-owner wave (or one half)
+  static constexpr int RPG = 16 / NW;   // rows per row-owner wave and row group
+  static constexpr int LDS_CAP = NW == 4 ? 80 * 1024 : 160 * 1024 * NW / (4 * OCC);
   static constexpr int REGION = RG * HP * 16 * 16;  // one fp32 term: [row group][HP heads][key] x 4 rows
   static constexpr int SCAL_BYTES = 2 * RC * 16 * 4;  // lse * log2(e) and D - dob: [term][head][row]
   static constexpr int BASE_BYTES = 2 * REGION + SCAL_BYTES;
@@ -904,17 +909,18 @@ struct Cols2Cfg {
   // row-major and transposed operand fragments are LDS reads; otherwise they
   // stream through registers and are transposed on the matrix core.
   static constexpr int QO_BYTES = 2 * HP * (D / 32) * 1024;
-  static constexpr bool QL = D % 32 == 0 && RC == 16 && BASE_BYTES + QO_BYTES <= 80 * 1024;
+  static constexpr bool QL = D % 32 == 0 && RC == 16 && BASE_BYTES + QO_BYTES <= LDS_CAP;
   static constexpr int LDS_BYTES = BASE_BYTES + (QL ? QO_BYTES : 0);
-  static constexpr bool FITS = LDS_BYTES <= 80 * 1024 && HP % 4 == 0;
+  static constexpr bool FITS = LDS_BYTES <= LDS_CAP && HP % NW == 0 && (NW == 4 || RC == 16);
 };
 
 
-template <int HP, int D, int C, int RC, int FL, int OCC>
-__global__ __launch_bounds__(256, OCC) void bwd_cols2_kernel(BwdParams prm) {
-  using Cfg = Cols2Cfg<HP, D, C, RC>;
+template <int HP, int D, int C, int RC, int FL, int OCC, int NW>
+__global__ __launch_bounds__(64 * NW, OCC) void bwd_cols2_kernel(BwdParams prm) {
+  using Cfg = Cols2Cfg<HP, D, C, RC, NW, OCC>;
   using DT = DTiles<D>;
-  constexpr int HW = Cfg::HW, NS = Cfg::NS, NCT = Cfg::NCT, NQ = DT::NQ, RGW = Cfg::RGW;
+  constexpr int HW = Cfg::HW, NS = Cfg::NS, NCT = Cfg::NCT, NQ = DT::NQ, RGW = Cfg::RGW, RPG = Cfg::RPG;
+  constexpr int NT = 64 * NW;
   constexpr bool QL = Cfg::QL;
   // TR: the transposed qt / dO reads in QoTile::tr_frag's order, free of
   // bank conflicts, with dk / dv regathered into 16-byte store order through
@@ -952,13 +958,13 @@ __global__ __launch_bounds__(256, OCC) void bwd_cols2_kernel(BwdParams prm) {
   bf16* dkg = reinterpret_cast<bf16*>(prm.dk);
   bf16* dvg = reinterpret_cast<bf16*>(prm.dv);
   if (event_refused(ev, eb)) {
-    fill_rows_nan<bf16, D>(rx, rx, k0, min(k0 + 16, len), H, tid, 256, dkg, nullptr);
-    fill_rows_nan<bf16, D>(rx, rx, k0, min(k0 + 16, len), H, tid, 256, dvg, nullptr);
+    fill_rows_nan<bf16, D>(rx, rx, k0, min(k0 + 16, len), H, tid, NT, dkg, nullptr);
+    fill_rows_nan<bf16, D>(rx, rx, k0, min(k0 + 16, len), H, tid, NT, dvg, nullptr);
     return;
   }
   if (k0 >= len) {
-    zero_tile_rows<bf16, D>(ev, rx, rx, k0, len, H, tid, dkg, nullptr);
-    zero_tile_rows<bf16, D>(ev, rx, rx, k0, len, H, tid, dvg, nullptr);
+    zero_tile_rows<bf16, D, NT>(ev, rx, rx, k0, len, H, tid, dkg, nullptr);
+    zero_tile_rows<bf16, D, NT>(ev, rx, rx, k0, len, H, tid, dvg, nullptr);
     return;
   }
   const bf16x4 id = ident_x16(g, n);
@@ -981,7 +987,10 @@ __global__ __launch_bounds__(256, OCC) void bwd_cols2_kernel(BwdParams prm) {
     for (int q = 0; q < NQ; ++q) dK[hl][q] = dV[hl][q] = zero4();
   }
 
-  // ---- row-owner: streamed rows 4 (RGW w + q') + r of each chunk ----
+  // ---- row-owner: streamed rows 4 rg + ro + r (r < RPG) of each chunk ----
+  // Row group of part q', and the wave's first row in it (0 unless eight
+  // waves share the groups in halves).
+  const int rg0 = NW == 4 ? RGW * w : w >> 1, ro = NW == 4 ? 0 : 2 * (w & 1);
   float4 pos_k = float4{0.f, 0.f, 0.f, 0.f};
   float fa[NCT], fb[NCT];
   if (use_e) {
@@ -1082,26 +1091,26 @@ __global__ __launch_bounds__(256, OCC) void bwd_cols2_kernel(BwdParams prm) {
   };
   // Row positions and the u / w~ rows of the row-owner part run one chunk
   // further ahead: they are needed first thing in a chunk.
-  bf16x4 ur[RGW][4][NCT], wr[RGW][4][NCT];
+  bf16x4 ur[RGW][RPG][NCT], wr[RGW][RPG][NCT];
   auto issue_rows = [&](int in, auto nf_tag) __attribute__((always_inline)) {
     constexpr bool NF = decltype(nf_tag)::value;
     if (use_e) {
 #pragma unroll
       for (int q2 = 0; q2 < RGW; ++q2) {
-        const int rg = RGW * w + q2;
+        const int rg = rg0 + q2;
         if constexpr (NF)
-          prow[q2] = pbuf.ldf4((4 * rg + g) * 16, in * 16);
+          prow[q2] = pbuf.ldf4((4 * rg + ro + g % RPG) * 16, in * 16);
         else
-          prow[q2] = pbuf.ldf4(min(in + 4 * rg + g, last) * 16, 0);
+          prow[q2] = pbuf.ldf4(min(in + 4 * rg + ro + g % RPG, last) * 16, 0);
         // Groups past the event reread its last group: their rows carry
         // P = 0 (lse = +inf) in the head-owner part.
         const int go = NF ? (int)(rg * ggrp) : (int)(min((in >> 2) + rg, glast) * ggrp);
         const int gso = NF ? (int)((in >> 2) * ggrp) * 2 : 0;
 #pragma unroll
-        for (int half = 0; half < 2; ++half)
+        for (int half = 0; half < RPG / 2; ++half)
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct) {
-            const int co = (go + uw_off(half, ct, n, g, 0, H, NCT)) * 2;
+            const int co = (go + uw_off(half + (ro >> 1), ct, n, g, 0, H, NCT)) * 2;
             if (attn) {
               const bf16x8 v = ubuf.ld128(co, gso);
               ur[q2][2 * half][ct] = lo4(v);
@@ -1133,12 +1142,12 @@ __global__ __launch_bounds__(256, OCC) void bwd_cols2_kernel(BwdParams prm) {
     if (use_e) {
 #pragma unroll
       for (int q2 = 0; q2 < RGW; ++q2) {
-        const int rg = RGW * w + q2;
+        const int rg = rg0 + q2;
         float xg[4];
         group_gather(pair_angle_unit(prow[q2], pos_k), xg);
-        f32x4 ue[4], we[4];
+        f32x4 ue[RPG], we[RPG];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < RPG; ++r) {
           bf16x4 ef[NCT];
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct) ef[ct] = embed_step<C>(xg[r], fa[ct], fb[ct], ct);
@@ -1155,8 +1164,13 @@ __global__ __launch_bounds__(256, OCC) void bwd_cols2_kernel(BwdParams prm) {
           // Heads past HP (lane groups g >= HP / 4) have no slot.
           const int so = ((rg * HP + 4 * g + e) * 16 + n) * 16;
           if (4 * g < HP) {
-            if (attn) *reinterpret_cast<f32x4*>(stU + so) = f32x4{ue[0][e], ue[1][e], ue[2][e], ue[3][e]};
-            if (act) *reinterpret_cast<f32x4*>(stW + so) = f32x4{we[0][e], we[1][e], we[2][e], we[3][e]};
+            if constexpr (RPG == 4) {
+              if (attn) *reinterpret_cast<f32x4*>(stU + so) = f32x4{ue[0][e], ue[1][e], ue[2][e], ue[3][e]};
+              if (act) *reinterpret_cast<f32x4*>(stW + so) = f32x4{we[0][e], we[1][e], we[2][e], we[3][e]};
+            } else {
+              if (attn) *reinterpret_cast<f32x2*>(stU + so + 4 * ro) = f32x2{ue[0][e], ue[1][e]};
+              if (act) *reinterpret_cast<f32x2*>(stW + so + 4 * ro) = f32x2{we[0][e], we[1][e]};
+            }
           }
         }
       }
@@ -1320,8 +1334,8 @@ __global__ __launch_bounds__(256, OCC) void bwd_cols2_kernel(BwdParams prm) {
       }
     }
   }
-  zero_tile_rows<bf16, D>(ev, rx, rx, k0, len, H, tid, dkg, nullptr);
-  zero_tile_rows<bf16, D>(ev, rx, rx, k0, len, H, tid, dvg, nullptr);
+  zero_tile_rows<bf16, D, NT>(ev, rx, rx, k0, len, H, tid, dkg, nullptr);
+  zero_tile_rows<bf16, D, NT>(ev, rx, rx, k0, len, H, tid, dvg, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1367,6 +1381,20 @@ struct Bwd2Pick {
   // against 0.437 ms; within 1 % elsewhere).
   static constexpr int ROWS_STATIC = NW == 8 ? 2 : ((HP % 8 == 0 && ROWS_W8X2) ? 3 : 1);
   static constexpr int COLS_STATIC = COLS_OCC3 ? 3 : 2;
+  // Eight cols-kernel waves per workgroup, each with half the heads of a
+  // four-wave one and two rows of each chunk (the same arithmetic), as waves
+  // per SIMD; 0: COLS_STATIC. At HP = 16 the four-wave instances spill from
+  // D = 48 on (D = 48, C = 16: 156 bytes a lane, D = C = 64: 764); eight waves
+  // in one workgroup per CU do not: B = 48, L = 768, lengths U{16..768}, D = 48,
+  // C = 16: 0.440 -> 0.312 ms, D = C = 48 -70 %, C = 64 1.463 -> 0.387, D = 64,
+  // C = 16 0.856 -> 0.345, D = C = 64 1.975 -> 0.491. At HP = 8 with D >= 48 and
+  // C <= 32 they run in two workgroups per CU, four waves per SIMD (B = 96,
+  // D = 64, C = 16: 0.314 -> 0.290, C = 32 0.365 -> 0.337, D = 48 -4 %). Elsewhere
+  // they lose (H = 8, D = C = 64: 3.01 -> 3.54 ms at B = 8, L = 4096; D = 32,
+  // C = 16 +9 %; H = 16, D = 32, C = 64 +16 %).
+  static constexpr int COLS_W8 = HP == 16 && D >= 48 && Cols2Cfg<HP, D, C, RC, 8, 2>::FITS             ? 2
+                                 : HP == 8 && D >= 48 && C <= 32 && Cols2Cfg<HP, D, C, RC, 8, 4>::FITS ? 4
+                                                                                                       : 0;
 };
 
 template <int HP, int D, int C, int NW, int WPE, bool KL>
@@ -1392,22 +1420,22 @@ int bwd2_launch_rows(const BwdParams& prm, hipStream_t stream, int g8, bool quer
   }
 }
 
-template <int HP, int D, int C, int OCC>
+template <int HP, int D, int C, int OCC, int NW>
 int bwd2_launch_cols(const BwdParams& prm, hipStream_t stream, int g8, bool query) {
   using P = Bwd2Pick<HP, D, C>;
-  using Cfg = Cols2Cfg<HP, D, C, P::RC>;
+  using Cfg = Cols2Cfg<HP, D, C, P::RC, NW, OCC>;
   if (query) return FST_OK;
   // One instance per bias-flag combination: a kernel reading the flags at
   // run time keeps both bias paths live and spills at the larger layouts.
   const int fl = prm.flags & 3;
-  auto kern = fl == 3   ? bwd_cols2_kernel<HP, D, C, P::RC, 3, OCC>
-              : fl == 1 ? bwd_cols2_kernel<HP, D, C, P::RC, 1, OCC>
-              : fl == 2 ? bwd_cols2_kernel<HP, D, C, P::RC, 2, OCC>
-                        : bwd_cols2_kernel<HP, D, C, P::RC, 0, OCC>;
+  auto kern = fl == 3   ? bwd_cols2_kernel<HP, D, C, P::RC, 3, OCC, NW>
+              : fl == 1 ? bwd_cols2_kernel<HP, D, C, P::RC, 1, OCC, NW>
+              : fl == 2 ? bwd_cols2_kernel<HP, D, C, P::RC, 2, OCC, NW>
+                        : bwd_cols2_kernel<HP, D, C, P::RC, 0, OCC, NW>;
   if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES) !=
       hipSuccess)
     return FST_ELAUNCH;
-  if (g8 > 0) hipLaunchKernelGGL(kern, dim3(g8), dim3(256), Cfg::LDS_BYTES, stream, prm);
+  if (g8 > 0) hipLaunchKernelGGL(kern, dim3(g8), dim3(64 * NW), Cfg::LDS_BYTES, stream, prm);
   return hipGetLastError() == hipSuccess ? FST_OK : FST_ELAUNCH;
 }
 
@@ -1463,12 +1491,15 @@ static int bwd2_launch_t(const BwdParams& prm, int which, hipStream_t stream, in
   if constexpr (!P::CC::FITS) {
     return FST_EUNSUPPORTED;
   } else {
+    if constexpr (P::COLS_W8 != 0)
+      if (!(f & (FST_PLAN_COLS_OCC2 | FST_PLAN_COLS_OCC3)))
+        return bwd2_launch_cols<HP, D, C, P::COLS_W8, 8>(prm, stream, g8, query);
     const int occ = (f & FST_PLAN_COLS_OCC2) ? 2 : (f & FST_PLAN_COLS_OCC3) ? 3 : P::COLS_STATIC;
     if (occ == 3) {
-      if constexpr (P::COLS_OCC3) return bwd2_launch_cols<HP, D, C, 3>(prm, stream, g8, query);
+      if constexpr (P::COLS_OCC3) return bwd2_launch_cols<HP, D, C, 3, 4>(prm, stream, g8, query);
       return FST_EUNSUPPORTED;
     }
-    return bwd2_launch_cols<HP, D, C, 2>(prm, stream, g8, query);
+    return bwd2_launch_cols<HP, D, C, 2, 4>(prm, stream, g8, query);
   }
 #endif
 }

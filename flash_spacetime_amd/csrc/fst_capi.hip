@@ -32,7 +32,8 @@ static int head_padding(int H) { return H <= 4 ? 4 : (H <= 8 ? 8 : (H <= 12 ? 12
 // Head padding of the bf16 rows kernel: where its four-wave instance would
 // spill, heads are padded to the next multiple of 8 so that it runs eight
 // waves (padded heads compute on a real head's data and store nothing). The
-// cols kernel keeps head_padding: the scratch between them is laid out by H.
+// scratch between the rows and cols kernel is laid out by H, so each pads as
+// it likes.
 // The eight-wave, one-workgroup plan (FST_PLAN_ROWS_W8) pads to a multiple
 // of 8 likewise; the four-wave plan and the eight-wave, two-workgroup plan
 // (which gives waves 4 to 7 one head fewer where 8 does not divide the
@@ -44,6 +45,18 @@ static int rows_head_padding(int dtype, int flags, int H, int D, int C) {
   if (flags & (FST_PLAN_ROWS_W4 | FST_PLAN_ROWS_W8X2)) return hp;
   if (hp % 8 != 0 && rows_wave_load(hp, D, C) >= 160) return hp + 4;
   return hp;
+}
+
+// Head padding of the bf16 cols kernel: 9 to 12 heads are padded to 16 where
+// the four-wave instance spills at 12 (D = 48, C >= 48) and the eight-wave one
+// at 16 does not (H = 12, D = 48, B = 48, L = 768, lengths U{16..768}: C = 64
+// 0.515 -> 0.359 ms, C = 48 0.367 -> 0.327; at D = 64 the four extra heads cost
+// more than the spills, C = 64 0.397 -> 0.454). Its plan bits name the
+// four-wave variants, at head_padding.
+static int cols_head_padding(int dtype, int flags, int H, int D, int C) {
+  const int hp = head_padding(H);
+  if (dtype != FST_BF16 || (flags & (FST_PLAN_COLS_OCC2 | FST_PLAN_COLS_OCC3))) return hp;
+  return hp == 12 && D == 48 && C >= 48 ? 16 : hp;
 }
 
 // fp32 frequency ladder exp(-i * ln(1e4) / (C/2)) evaluated with the same
@@ -543,7 +556,7 @@ static int bwd_layout(int dtype, int flags, int B, int H, int L, int T, int D, i
   BwdParams dummy;
   std::memset(&dummy, 0, sizeof(dummy));
   dummy.flags = flags;  // the queries resolve the plan bits
-  const int HP = head_padding(H), HPR = rows_head_padding(dtype, flags, H, D, C);
+  const int HP = cols_head_padding(dtype, flags, H, D, C), HPR = rows_head_padding(dtype, flags, H, D, C);
   if (fn(dummy, 0, HPR, C, nullptr, 0, true, &lay.rows_r) != FST_OK || lay.rows_r <= 0) return FST_EUNSUPPORTED;
   if (fn(dummy, 1, HP, C, nullptr, 0, true, &lay.rows_c) != FST_OK || lay.rows_c <= 0) return FST_EUNSUPPORTED;
   const bool packed = flags & FST_PACKED;
@@ -902,7 +915,7 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
   freq_table(C, prm.freq);
 
   bwd_dispatch_fn fn = bwd_table(dtype, D);
-  const int HP = head_padding(H), HPR = rows_head_padding(dtype, flags, H, D, C);
+  const int HP = cols_head_padding(dtype, flags, H, D, C), HPR = rows_head_padding(dtype, flags, H, D, C);
   int dummy_rows = 0;
   if (phases & FST_PHASE_BWD_ROWS) {
     rc = fn(prm, 0, HPR, C, st, (int)lay.grid_r, false, &dummy_rows);

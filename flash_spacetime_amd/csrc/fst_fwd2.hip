@@ -34,33 +34,37 @@
 
 namespace fst {
 
-template <int HP, int D, int C, int KC, int OCC>
+// NW waves of 64 lanes per workgroup, OCC waves per SIMD the register and LDS
+// plan is built for (4 OCC / NW workgroups per CU).
+template <int HP, int D, int C, int KC, int OCC, int NW = 4>
 struct Fwd2Cfg {
-  static constexpr int HW = HP / 4;  // heads per wave
+  static constexpr int HW = HP / NW;  // heads per wave
+  static constexpr int RPW = 16 / NW;  // rows per row-owner wave
+  static constexpr int WG_PER_CU = 4 * OCC / NW;
   static constexpr int NS = KC / 16;  // 16-key subtiles per chunk
   static constexpr int NCT = C / 16;  // channel steps
   static constexpr int E_BYTES = ETile<C, KC>::BYTES;
   static constexpr int STAGE_BYTES = (KC / 4) * 16 * 16 * 16;  // fp32 u.E of KC keys per (row, head)
-  static constexpr int SCAL_BYTES = 16 * 17 * 4 + 16;  // rescale factors, then one flag per wave
+  static constexpr int SCAL_BYTES = 16 * 17 * 4 + 4 * NW;  // rescale factors, then one flag per wave
   static constexpr int BASE_BYTES = E_BYTES + STAGE_BYTES + SCAL_BYTES;
   // VL: each chunk's V rows go straight to LDS (QoTile blocks, one per head
   // and 32-feature part) and are read transposed there, where D is a multiple
   // of 32, the chunk 16 keys and the blocks fit the occupancy's LDS share.
   static constexpr int V_BYTES = HP * (D / 32) * 1024;
-  static constexpr bool VL = D % 32 == 0 && KC == 16 && BASE_BYTES + V_BYTES <= (160 / OCC) * 1024;
+  static constexpr bool VL = D % 32 == 0 && KC == 16 && BASE_BYTES + V_BYTES <= 160 * 1024 / WG_PER_CU;
   static constexpr int LDS_BYTES = BASE_BYTES + (VL ? V_BYTES : 0);
-  // OCC: workgroups per CU the register and LDS plan is built for.
-  static constexpr bool FITS = LDS_BYTES <= (160 / OCC) * 1024 && HP % 4 == 0 && (KC == 16 || KC == 32);
+  static constexpr bool FITS = (NW == 4 || NW == 8) && HP % NW == 0 && (KC == 16 || KC == 32) &&
+                               LDS_BYTES <= 160 * 1024 / WG_PER_CU;
 };
 
 constexpr float kRescaleLog2 = 8.f;
 
-template <int HP, int D, int C, int KC, int OCC, int FL>
-__global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
-  using Cfg = Fwd2Cfg<HP, D, C, KC, OCC>;
+template <int HP, int D, int C, int KC, int OCC, int NW, int FL>
+__global__ __launch_bounds__(64 * NW, OCC) void fwd2_kernel(FwdParams prm) {
+  using Cfg = Fwd2Cfg<HP, D, C, KC, OCC, NW>;
   using ET = ETile<C, KC>;
   using DT = DTiles<D>;
-  constexpr int HW = Cfg::HW, NS = Cfg::NS, NCT = Cfg::NCT, NQ = DT::NQ;
+  constexpr int HW = Cfg::HW, NS = Cfg::NS, NCT = Cfg::NCT, NQ = DT::NQ, RPW = Cfg::RPW, NT = 64 * NW;
   constexpr bool VL = Cfg::VL;
   constexpr int NP = D / 32;  // 32-feature parts of a row (VL)
   extern __shared__ __align__(16) unsigned char smem[];
@@ -87,11 +91,11 @@ __global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
   const int last = len - 1;
   bf16* outg = reinterpret_cast<bf16*>(prm.out);
   if (event_refused(prm.ev, eb)) {
-    fill_rows_nan<bf16, D>(ra, ra, i0, min(i0 + 16, len), H, tid, 256, outg, prm.lse);
+    fill_rows_nan<bf16, D>(ra, ra, i0, min(i0 + 16, len), H, tid, NT, outg, prm.lse);
     return;
   }
   if (i0 >= len) {  // a tile of padding rows only
-    zero_tile_rows<bf16, D>(prm.ev, ra, ra, i0, len, H, tid, outg, prm.lse);
+    zero_tile_rows<bf16, D, NT>(prm.ev, ra, ra, i0, len, H, tid, outg, prm.lse);
     return;
   }
 
@@ -118,23 +122,25 @@ __global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
     qf[hl].load(qg + rx.off(hq, row_ok ? my_row : last, D), g);
   }
 
-  // ---- row-owner state: rows i0 + 4w + r, heads on lane n ----
+  // ---- row-owner state: rows i0 + row0 + r (r < RPW), heads on lane n ----
+  const int row0 = RPW * w;
   WSlots<D, C> wv;
-  SlotRow<D> xq[4];
+  SlotRow<D> xq[RPW];
   if (attn) {
     wv.load(prm.weight, g, n);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = i0 + 4 * w + r;
+    for (int r = 0; r < RPW; ++r) {
+      const int row = i0 + row0 + r;
       xq[r].load(qg + rx.off(0, row < len ? row : last, D), rx.hs * D, row < len && n < H, g, n);
     }
   }
-  // Angle lane assignment: lane (g, n) evaluates row i0 + 4w + g against key
-  // j0 + 16 s + n; the four rows are then gathered into every lane group.
+  // Angle lane assignment: lane (g, n) evaluates row i0 + row0 + g % RPW
+  // against key j0 + 16 s + n (with two rows a wave, lane groups 2 and 3 repeat
+  // 0 and 1); the rows are then gathered into every lane group.
   float4 pos_i = float4{0.f, 0.f, 0.f, 0.f};
   float fa[NCT], fb[NCT];
   if (use_e) {
-    const int row = i0 + 4 * w + g;
+    const int row = i0 + row0 + g % RPW;
     pos_i = ra.pos(prm.ev.pos4, row < len ? row : last);
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) {
@@ -227,13 +233,13 @@ __global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
     lsum[hl] = 0.f;
     mref[hl] = -INFINITY;
   }
-  bf16x4 uf[4][NCT];
-  f32x4 AE[4][NCT];
+  bf16x4 uf[RPW][NCT];
+  f32x4 AE[RPW][NCT];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
+  for (int r = 0; r < RPW; ++r) {
     if (attn) {
       // u^T[slot][h] = scale sum_d W[d][channel(slot)] q[h][d] (project_loaded).
-      project_loaded<D, C>(xq[r], i0 + 4 * w + r < len && n < H, prm.scale, wv, uf[r]);
+      project_loaded<D, C>(xq[r], i0 + row0 + r < len && n < H, prm.scale, wv, uf[r]);
     } else {
 #pragma unroll
       for (int ct = 0; ct < NCT; ++ct) uf[r][ct] = bf16x4{};
@@ -247,7 +253,7 @@ __global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
     constexpr bool TAIL = decltype(tail_tag)::value;
     issue_v(j0);  // lands during the row-owner part
 
-    // ---- row-owner: E of rows 4w..4w+3 x KC keys; u.E staged ----
+    // ---- row-owner: E of its rows x KC keys; u.E staged ----
     if (use_e) {
       float xg[NS][4];
 #pragma unroll
@@ -256,20 +262,20 @@ __global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
       // epilogue back).
       if (decltype(next_tag)::value || j0 + KC < len) issue_pos(j0 + KC, next_tag);
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int r = 0; r < RPW; ++r)
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
           bf16x4 ef[NCT];
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct) {
             ef[ct] = embed_step<C>(xg[s][r], fa[ct], fb[ct], ct);
-            if (act) ET::store(Es, 4 * w + r, ct, 16 * s + n, g, ef[ct]);
+            if (act) ET::store(Es, row0 + r, ct, 16 * s + n, g, ef[ct]);
           }
           if (attn) {
             f32x4 ue = zero4();
 #pragma unroll
             for (int ct = 0; ct < NCT; ++ct) ue = mfma_x16(ef[ct], uf[r][ct], ue);
-            *reinterpret_cast<f32x4*>(stage + stage_off(4 * s + g, 4 * w + r, n)) = ue;
+            *reinterpret_cast<f32x4*>(stage + stage_off(4 * s + g, row0 + r, n)) = ue;
           }
           // One (row, subtile) at a time: the scheduler's own interleaving of
           // the rows measured 2 % slower.
@@ -396,24 +402,33 @@ __global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
 
     // ---- row-owner: A = alpha A + E^T P ----
     if (act) {
-      const int4 fl = *reinterpret_cast<const int4*>(rflag);
-      if (__builtin_amdgcn_readfirstlane(fl.x | fl.y | fl.z | fl.w)) {
+      int fl[NW], any = 0;
+#pragma unroll
+      for (int k = 0; k < NW; k += 4) {
+        const int4 f4 = *reinterpret_cast<const int4*>(rflag + k);
+        fl[k] = f4.x, fl[k + 1] = f4.y, fl[k + 2] = f4.z, fl[k + 3] = f4.w;
+        any |= f4.x | f4.y | f4.z | f4.w;
+      }
+      if (__builtin_amdgcn_readfirstlane(any)) {
         // Rare: some head-owner moved its reference m this chunk. (The empty
         // volatile asm keeps this a branch rather than selects.)
         __asm__ volatile("");
         const int ow = n / HW;  // the wave that owns head n
-        const bool fresh = n < H && (ow == 0 ? fl.x : ow == 1 ? fl.y : ow == 2 ? fl.z : fl.w) != 0;
+        int fw = fl[NW - 1];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float al = *reinterpret_cast<const float*>(scal + scal_off(4 * w + r, n));
+        for (int k = 0; k < NW - 1; ++k) fw = ow == k ? fl[k] : fw;
+        const bool fresh = n < H && fw != 0;
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
+          const float al = *reinterpret_cast<const float*>(scal + scal_off(row0 + r, n));
           const float alpha = fresh ? al : 1.f;
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct) AE[r][ct] = AE[r][ct] * alpha;
         }
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int il = 4 * w + r;
+      for (int r = 0; r < RPW; ++r) {
+        const int il = row0 + r;
         JFrag<bf16, NS> pr;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
@@ -489,10 +504,10 @@ __global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
   // sum_slot W[d, channel(slot)] A^T_i[slot, h] on bf16 MFMA over the two
   // parts of each factor (W and A to 16 bits) and stages it; the head-owner
   // forms out = (O + o2) / l + b in place.
-  bf16x4 aeh[4][NCT], ael[4][NCT];
+  bf16x4 aeh[RPW][NCT], ael[RPW][NCT];
   if (act) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < RPW; ++r)
 #pragma unroll
       for (int ct = 0; ct < NCT; ++ct) split4(AE[r][ct], aeh[r][ct], ael[r][ct]);
   }
@@ -502,11 +517,11 @@ __global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
       if constexpr (!WPRE) load_w(q);
       __syncthreads();  // previous round (or the last chunk) done with the stage
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
+      for (int r = 0; r < RPW; ++r) {
         f32x4 acc = zero4();
 #pragma unroll
         for (int ct = 0; ct < NCT; ++ct) acc = mma_split(wh[q][ct], wl[q][ct], aeh[r][ct], ael[r][ct], acc);
-        *reinterpret_cast<f32x4*>(stage + stage_off(g, 4 * w + r, n)) = acc;
+        *reinterpret_cast<f32x4*>(stage + stage_off(g, row0 + r, n)) = acc;
       }
       __syncthreads();
     }
@@ -536,7 +551,7 @@ __global__ __launch_bounds__(256, OCC) void fwd2_kernel(FwdParams prm) {
     }
   }
 
-  zero_tile_rows<bf16, D>(prm.ev, ra, ra, i0, len, H, tid, outg, prm.lse);
+  zero_tile_rows<bf16, D, NT>(prm.ev, ra, ra, i0, len, H, tid, outg, prm.lse);
 }
 
 template <int HP, int D, int C>
@@ -557,6 +572,21 @@ struct Fwd2Pick {
   // 32-key chunks (FST_PLAN_FWD_KC32) at two workgroups per CU, where their
   // LDS plan fits and the lane state is that of the small layouts.
   static constexpr bool KC32 = OK && Fwd2Cfg<HP, D, C, 32, 2>::FITS && rows_wave_load(HP, D, C) < 160;
+  // Eight waves per workgroup, each with half the heads and rows of a
+  // four-wave one (the same arithmetic), as waves per SIMD; 0: four waves.
+  // At HP = 16 the four-wave instances spill from (HP / 4) D + 3 C = 336 on
+  // with D >= 48 (D = C = 48: 176 bytes a lane, D = C = 64: 540); eight waves
+  // in one workgroup per CU do not: B = 48, L = 768, lengths U{16..768}, D = 48,
+  // C = 64: 0.906 -> 0.406 ms, D = C = 64: 1.472 -> 0.387, D = C = 48 -25 %,
+  // D = 64, C = 32 -4 %. Below that line they lose (D = 48, C = 16: 0.215 ->
+  // 0.288 ms; C = 32 equal; D = 32, C = 64: 0.250 -> 0.273). At D = 32, C = 16
+  // eight waves in two workgroups per CU (116 registers, four waves per SIMD)
+  // measured 0.241 -> 0.226 ms; every other light shape lost (H = 8, D = 32,
+  // C = 16: 0.147 -> 0.180).
+  static constexpr int W8 = HP != 16                                     ? 0
+                            : D >= 48 && rows_wave_load(HP, D, C) >= 336 ? (Fwd2Cfg<HP, D, C, KC, 2, 8>::FITS ? 2 : 0)
+                            : D == 32 && C == 16                         ? (Fwd2Cfg<HP, D, C, KC, 4, 8>::FITS ? 4 : 0)
+                                                                         : 0;
   // Occupancy and key-chunk variants a caller may choose instead (the plan
   // bits of include/flash_spacetime.h); the occupancy variants compute every
   // row with the same arithmetic.
@@ -565,32 +595,33 @@ struct Fwd2Pick {
                                   : 0;
 };
 
-template <int HP, int D, int C, int KC, int OCC>
+template <int HP, int D, int C, int KC, int OCC, int NW = 4>
 int fwd2_launch_occ(const FwdParams& prm, hipStream_t stream, int grid, bool query) {
-  using Cfg = Fwd2Cfg<HP, D, C, KC, OCC>;
+  using Cfg = Fwd2Cfg<HP, D, C, KC, OCC, NW>;
   using P = Fwd2Pick<HP, D, C>;
-  constexpr bool OFFERED = KC == 16 ? (OCC == 2 ? P::OCC2 : P::OCC3) : (P::KC32 && OCC == 2);
+  constexpr bool OFFERED = NW == 8 ? P::W8 == OCC : KC == 16 ? (OCC == 2 ? P::OCC2 : P::OCC3) : (P::KC32 && OCC == 2);
   if constexpr (!Cfg::FITS || !OFFERED) {
     return FST_EUNSUPPORTED;
   } else {
     if (query) return FST_OK;
     // Both bias flags (the operators' default) run an instance with the flags
     // fixed at compile time; other combinations read them at run time.
-    auto kern = (prm.flags & 3) == 3 ? fwd2_kernel<HP, D, C, KC, OCC, 3> : fwd2_kernel<HP, D, C, KC, OCC, -1>;
+    auto kern = (prm.flags & 3) == 3 ? fwd2_kernel<HP, D, C, KC, OCC, NW, 3> : fwd2_kernel<HP, D, C, KC, OCC, NW, -1>;
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES) !=
         hipSuccess)
       return FST_ELAUNCH;
     // The grid is rounded up to a multiple of 64 for the XCD schedules
     // (tile_block); logical blocks past the work list exit at once.
     const int g8 = (grid + 63) & ~63;
-    if (grid > 0) hipLaunchKernelGGL(kern, dim3(g8), dim3(256), Cfg::LDS_BYTES, stream, prm);
+    if (grid > 0) hipLaunchKernelGGL(kern, dim3(g8), dim3(64 * NW), Cfg::LDS_BYTES, stream, prm);
     return hipGetLastError() == hipSuccess ? FST_OK : FST_ELAUNCH;
   }
 }
 
 // Launches (or, with query, only checks) the variant the plan bits of
-// prm.flags name: an empty occupancy group takes the static occupancy (two
-// with 32-key chunks), an empty key-chunk group 16 keys.
+// prm.flags name: an empty occupancy group takes the static waves and
+// occupancy (four waves, two workgroups per CU with 32-key chunks), an empty
+// key-chunk group 16 keys. The occupancy bits name the four-wave variants.
 template <int HP, int D, int C>
 int fwd2_launch_t(const FwdParams& prm, hipStream_t stream, int grid, bool query) {
   using P = Fwd2Pick<HP, D, C>;
@@ -599,6 +630,9 @@ int fwd2_launch_t(const FwdParams& prm, hipStream_t stream, int grid, bool query
   } else {
     const bool kc32 = prm.flags & FST_PLAN_FWD_KC32;
     const int occ = (prm.flags & FST_PLAN_FWD_OCC2) ? 2 : (prm.flags & FST_PLAN_FWD_OCC3) ? 3 : (kc32 ? 2 : P::OCC);
+    if constexpr (P::W8 != 0)
+      if (!(prm.flags & (FST_PLAN_FWD_OCC2 | FST_PLAN_FWD_OCC3)) && !kc32)
+        return fwd2_launch_occ<HP, D, C, 16, P::W8, 8>(prm, stream, grid, query);
     if (kc32) return occ == 2 ? fwd2_launch_occ<HP, D, C, 32, 2>(prm, stream, grid, query) : FST_EUNSUPPORTED;
     if (occ == 3) return fwd2_launch_occ<HP, D, C, 16, 3>(prm, stream, grid, query);
     return fwd2_launch_occ<HP, D, C, 16, 2>(prm, stream, grid, query);
