@@ -151,7 +151,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_rows_kernel(Bwd
   const int tile = wave / NW, ws = wave % NW;
 
   EventBlock eb;
-  if (!locate_block(prm.ev, blockIdx.x, eb)) return;
+  if (!locate_block(prm.ev, Cfg::ROWS, blockIdx.x, eb)) return;
   const int len = eb.len;
   const int H = prm.H;
   const bool attn = prm.flags & FST_ATTN_BIAS;
@@ -747,7 +747,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_cols_kernel(Bwd
   EventSpec ev = prm.ev;
   ev.blkcum = prm.blkcum_cols;
   EventBlock eb;
-  if (!locate_block(ev, blockIdx.x, eb)) return;
+  if (!locate_block(ev, Cfg::KEYS, blockIdx.x, eb)) return;
   const int len = eb.len;
   const int H = prm.H;
   const bool attn = prm.flags & FST_ATTN_BIAS;

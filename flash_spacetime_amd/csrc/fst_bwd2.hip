@@ -137,7 +137,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void bwd_rows2_kernel(BwdParams prm) 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
   EventBlock eb;
-  if (!tile_block(prm.ev, blockIdx.x, eb)) return;
+  if (!tile_block(prm.ev, !prm.ev.packed, blockIdx.x, eb)) return;
   const int len = eb.len;
   const int H = prm.H;
   // FL >= 0: the bias flags fixed at compile time; -1: read at run time.
@@ -153,9 +153,8 @@ __global__ __launch_bounds__(64 * NW, WPE) void bwd_rows2_kernel(BwdParams prm) 
   // empty padded event owns one slot, written as zeros); tiles of padding
   // rows past an event's last tile own none.
   const int nbv = len > 0 ? (len + 15) / 16 : (prm.ev.packed ? 0 : 1);
-  // The tile's slot in the work list (read once: after the prologue's
-  // stores it would be read again, waiting for every load before it).
-  const long tslot = (long)prm.ev.blkcum[eb.b] + eb.blk;
+  // The tile's slot in the work list.
+  const long tslot = (long)eb.tile0 + eb.blk;
   float* part = eb.blk < nbv ? prm.dw_part + tslot * DCW : nullptr;
   if (event_refused(prm.ev, eb)) {
     fill_rows_nan<bf16, D>(rx, ra, i0, min(i0 + 16, len), H, tid, NT, dqg, prm.rowsum);
@@ -942,9 +941,9 @@ __global__ __launch_bounds__(64 * NW, OCC) void bwd_cols2_kernel(BwdParams prm) 
   EventSpec ev = prm.ev;
   ev.blkcum = prm.blkcum_cols;
   ev.scum = prm.scum_cols;
-  ev.vp = nullptr;  // the interleaved schedule (the padding-last one is the rows kernel's)
   EventBlock eb;
-  if (!tile_block(ev, blockIdx.x, eb)) return;
+  // The interleaved schedule (the padding-last one is the rows kernel's).
+  if (!tile_block(ev, false, blockIdx.x, eb)) return;
   const int len = eb.len;
   const int H = prm.H;
   // FL >= 0: the bias flags fixed at compile time; -1: read at run time.
@@ -1014,7 +1013,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void bwd_cols2_kernel(BwdParams prm) 
   // u / w~ in the row-group layout the rows kernel writes (uw_off): the
   // event's groups start at 4 x its first tile in the rows work list.
   const long ggrp = uw_group_elems(H, NCT);
-  const long cbase = (long)prm.ev.blkcum[eb.b] * 4 * ggrp;
+  const long cbase = (long)eb.tile0 * 4 * ggrp;
   const int glast = (len - 1) >> 2;  // last row group of the event
   const unsigned cbytes = (unsigned)((long)(glast + 1) * ggrp * 2);
   const Buf ubuf(reinterpret_cast<const bf16*>(prm.u) + cbase, cbytes),

@@ -502,20 +502,38 @@ static bwd_dispatch_fn bwd_table(int dtype, int D) {
 // dW / db from the per-block partials of the rows kernel, in two fixed-order
 // stages so the result does not depend on scheduling: stage 1 sums runs of
 // kRedSeg consecutive blocks per column (coalesced over the columns), stage
-// 2 sums the run totals in order.
+// 2 sums the run totals in four interleaved sums added in order.
 constexpr int kRedSeg = 64;
 
-__global__ __launch_bounds__(256) void dw_reduce_seg_kernel(const float* part, const int32_t* blkcum, int B,
-                                                            int ncol, float* seg) {
-  const int nblk = blkcum[B];
-  const int col = blockIdx.x * 256 + threadIdx.x;
-  if (col >= ncol) return;
-  const long w0 = (long)blockIdx.y * kRedSeg;
+// Blocks of the call's work list (of `rows` rows).
+__device__ __forceinline__ int total_blocks(const EventSpec& ev, int rows) {
+  if (!ev.inl) return ev.blkcum[ev.B];
+  return __builtin_amdgcn_readlane(InlineList(ev, rows).incl, 63);
+}
+
+// Blocks [64 s, 64 s + 64) of column col, in order.
+__device__ __forceinline__ float run_sum(const float* part, int nblk, int ncol, int s, int col) {
+  const long w0 = (long)s * kRedSeg;
   const long w1 = w0 + kRedSeg < nblk ? w0 + kRedSeg : nblk;
   float acc = 0.f;
 #pragma unroll 8
   for (long w = w0; w < w1; ++w) acc += part[w * ncol + col];
-  seg[(long)blockIdx.y * ncol + col] = acc;
+  return acc;
+}
+
+__global__ __launch_bounds__(256) void dw_reduce_seg_kernel(const float* part, EventSpec ev, int rows, int ncol,
+                                                            float* seg) {
+  const int nblk = total_blocks(ev, rows);
+  const int col = blockIdx.x * 256 + threadIdx.x;
+  if (col >= ncol) return;
+  seg[(long)blockIdx.y * ncol + col] = run_sum(part, nblk, ncol, blockIdx.y, col);
+}
+
+__device__ __forceinline__ void store_dw(float acc, int e, int DC, float* dw, float* db) {
+  if (e < DC)
+    dw[e] = acc;
+  else if (db)
+    db[e - DC] = acc;
 }
 
 // Stage 2: a workgroup per 64 columns; thread (q, c) sums runs q, q + 4, ...
@@ -533,11 +551,32 @@ __global__ __launch_bounds__(256) void dw_reduce_final_kernel(const float* seg, 
   part[q][c] = acc;
   __syncthreads();
   if (q != 0 || e >= DC + D) return;
-  acc = ((part[0][c] + part[1][c]) + part[2][c]) + part[3][c];
-  if (e < DC)
-    dw[e] = acc;
-  else if (db)
-    db[e - DC] = acc;
+  store_dw(((part[0][c] + part[1][c]) + part[2][c]) + part[3][c], e, DC, dw, db);
+}
+
+// Both stages in one launch for at most kRedOne runs (1024 blocks): a
+// workgroup per 64 columns, one thread per (run, column), the run totals
+// exchanged through LDS and added in the two-launch order (bit for bit the
+// same sums). A launch less on calls whose kernels take 15 to 60 us; with
+// more runs the two-launch form spreads them over more workgroups.
+constexpr int kRedOne = 16;
+__global__ __launch_bounds__(64 * kRedOne) void dw_reduce_one_kernel(const float* part, EventSpec ev, int rows,
+                                                                     int nseg, int DC, int D, int use_e, float* dw,
+                                                                     float* db) {
+  __shared__ float run[kRedOne][64];
+  const int c = threadIdx.x & 63, s = threadIdx.x >> 6;
+  const int e = blockIdx.x * 64 + c;
+  const int nblk = total_blocks(ev, rows);  // by whole waves
+  if (s < nseg) run[s][c] = use_e && e < DC + D ? run_sum(part, nblk, DC + D, s, e) : 0.f;
+  __syncthreads();
+  if (s != 0 || e >= DC + D) return;
+  float q4[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    q4[q] = 0.f;
+    for (int k = q; k < nseg; k += 4) q4[q] += run[k][c];
+  }
+  store_dw(((q4[0] + q4[1]) + q4[2]) + q4[3], e, DC, dw, db);
 }
 
 __global__ __launch_bounds__(256) void fill_zero_kernel(float* p, int n) {
@@ -694,7 +733,10 @@ int fst_forward_phases(int phases, int dtype, int flags, int B, int H, int L, in
 
   const WorkList wl = worklist_at(workspace, B);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (phases & FST_PHASE_WORKLIST) {
+  // A whole call of few events needs no work list (InlineList); phases run
+  // one by one keep it.
+  const bool inl = B <= kInlineEvents && phases == FST_FWD_ALL;
+  if ((phases & FST_PHASE_WORKLIST) && !inl) {
     if (launch_worklist(lens, packed, B, L, T, rows, wl.blkcum, 0, nullptr, wl.perm, wl.scum, nullptr, wl.cus,
                         wl.status, st) != FST_OK)
       return fail(FST_ELAUNCH, "work-list kernel launch failed");
@@ -702,11 +744,14 @@ int fst_forward_phases(int phases, int dtype, int flags, int B, int H, int L, in
 
   if (!(phases & FST_PHASE_FWD)) return FST_OK;
 
-  prm.ev.lens = packed ? wl.cus : lens;
-  prm.ev.blkcum = wl.blkcum;
-  prm.ev.perm = wl.perm;
-  prm.ev.scum = packed ? wl.scum : nullptr;
-  prm.ev.status = wl.status;
+  prm.ev.inl = inl ? 1 : 0;
+  prm.ev.lens = packed && !inl ? wl.cus : lens;
+  if (!inl) {
+    prm.ev.blkcum = wl.blkcum;
+    prm.ev.perm = wl.perm;
+    prm.ev.scum = packed ? wl.scum : nullptr;
+    prm.ev.status = wl.status;
+  }
   prm.ev.max_len = max_event_len(dtype, flags, H, D, C);
   prm.ev.pos4 = reinterpret_cast<const float4*>(pos4);
   prm.ev.B = B;
@@ -863,7 +908,8 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
   // The bf16 rows kernel's padding-last schedule (16-row tiles, padded events).
   int32_t* vp = (dtype == FST_BF16 && !packed && lay.rows_r == 16) ? reinterpret_cast<int32_t*>(ws + lay.off_vp)
                                                                     : nullptr;
-  if (phases & FST_PHASE_WORKLIST) {
+  const bool inl = B <= kInlineEvents && phases == FST_BWD_ALL;  // as in the forward
+  if ((phases & FST_PHASE_WORKLIST) && !inl) {
     if (launch_worklist(lens, packed, B, L, T, lay.rows_r, wr.blkcum, lay.rows_c, wc.blkcum, wr.perm, wr.scum,
                         wc.scum, wr.cus, wr.status, st, vp) != FST_OK)
       return fail(FST_ELAUNCH, "work-list kernel launch failed");
@@ -871,12 +917,15 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
 
   BwdParams prm;
   std::memset(&prm, 0, sizeof(prm));
-  prm.ev.lens = packed ? wr.cus : lens;
-  prm.ev.blkcum = wr.blkcum;
-  prm.ev.perm = wr.perm;
-  prm.ev.scum = packed ? wr.scum : nullptr;
-  prm.ev.vp = vp;
-  prm.ev.status = wr.status;
+  prm.ev.inl = inl ? 1 : 0;
+  prm.ev.lens = packed && !inl ? wr.cus : lens;
+  if (!inl) {
+    prm.ev.blkcum = wr.blkcum;
+    prm.ev.perm = wr.perm;
+    prm.ev.scum = packed ? wr.scum : nullptr;
+    prm.ev.vp = vp;
+    prm.ev.status = wr.status;
+  }
   prm.ev.max_len = max_event_len(dtype, flags, H, D, C);
   prm.ev.pos4 = reinterpret_cast<const float4*>(pos4);
   prm.ev.B = B;
@@ -886,8 +935,8 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
   prm.ev.packed = packed ? 1 : 0;
   prm.ev.tokmajor = (packed || (flags & FST_TOKEN_MAJOR)) ? 1 : 0;
   prm.ev.xmul = (flags & FST_QKV_INTERLEAVED) ? 3 : 1;
-  prm.blkcum_cols = wc.blkcum;
-  prm.scum_cols = packed ? wc.scum : nullptr;
+  prm.blkcum_cols = inl ? nullptr : wc.blkcum;
+  prm.scum_cols = packed && !inl ? wc.scum : nullptr;
   prm.H = H;
   prm.flags = flags;
   prm.scale = scale;
@@ -930,11 +979,16 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
     const int ncol = DC + D;
     float* seg = reinterpret_cast<float*>(ws + lay.off_seg);
     if (lay.nseg > 65535) return fail(FST_EUNSUPPORTED, "problem too large for the dW reduction");
-    if (use_w && lay.nseg > 0)
-      hipLaunchKernelGGL(dw_reduce_seg_kernel, dim3((ncol + 255) / 256, (unsigned)lay.nseg), dim3(256), 0, st,
-                         prm.dw_part, wr.blkcum, B, ncol, seg);
-    hipLaunchKernelGGL(dw_reduce_final_kernel, dim3((ncol + 63) / 64), dim3(256), 0, st, seg, (int)lay.nseg, DC,
-                       D, use_w ? 1 : 0, dweight, dbias);
+    if (lay.nseg <= kRedOne) {
+      hipLaunchKernelGGL(dw_reduce_one_kernel, dim3((ncol + 63) / 64), dim3(64 * kRedOne), 0, st, prm.dw_part, prm.ev,
+                         lay.rows_r, (int)lay.nseg, DC, D, use_w ? 1 : 0, dweight, dbias);
+    } else {
+      if (use_w)
+        hipLaunchKernelGGL(dw_reduce_seg_kernel, dim3((ncol + 255) / 256, (unsigned)lay.nseg), dim3(256), 0, st,
+                           prm.dw_part, prm.ev, lay.rows_r, ncol, seg);
+      hipLaunchKernelGGL(dw_reduce_final_kernel, dim3((ncol + 63) / 64), dim3(256), 0, st, seg, (int)lay.nseg, DC,
+                         D, use_w ? 1 : 0, dweight, dbias);
+    }
     if (hipGetLastError() != hipSuccess) return fail(FST_ELAUNCH, "dW reduction launch failed");
   }
   return FST_OK;

@@ -97,7 +97,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void fwd_kernel(FwdParam
 
   // ---- work item: (event, row block) from the per-event block prefix ----
   EventBlock eb;
-  if (!locate_block(prm.ev, blockIdx.x, eb)) return;
+  if (!locate_block(prm.ev, Cfg::ROWS, blockIdx.x, eb)) return;
   const int len = eb.len;
   const int H = prm.H;
   const bool attn = prm.flags & FST_ATTN_BIAS;

@@ -26,10 +26,17 @@ struct EventSpec {
   int tokmajor;           // rows of one token's heads are adjacent (packed, or padded token-major)
   int xmul;               // 3: q, k, v (and dq, dk, dv) interleaved per token as [.., 3, H, X]; else 1
   int max_len;            // longest event whose rows of all heads span less than 2^31 bytes
+  // No work list: lens are the caller's (the raw cu_seqlens when packed) and
+  // every workgroup forms the lists it needs itself (InlineList); blkcum,
+  // perm, scum, vp and status are null. Calls of up to kInlineEvents events.
+  int inl;
 };
 
+// tile0: the event's first block in the work list (blkcum[b]); bad: the
+// call's packed offsets are malformed.
 struct EventBlock {
-  int b, blk, len, tok0;
+  int b, blk, len, tok0, tile0;
+  bool bad;
 };
 
 // Row addressing of one event. Offsets are in elements of a row of width X.
@@ -68,7 +75,7 @@ __device__ __forceinline__ void event_range(const EventSpec& ev, int b, int& tok
 // rows of all heads span 2^31 bytes or more, past the 32-bit byte offsets of
 // the buffer loads (which would read zeros there).
 __device__ __forceinline__ bool event_refused(const EventSpec& ev, const EventBlock& eb) {
-  return (ev.status && *ev.status != 0) || eb.len > ev.max_len;
+  return eb.bad || (ev.status && *ev.status != 0) || eb.len > ev.max_len;
 }
 
 // NaN into rows [r0, r1) of every head of a refused event: out (rows of
@@ -109,13 +116,90 @@ __device__ __forceinline__ int wave_last_le(int n, int t, F key) {
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
-// Work item of workgroup w: the event whose blocks hold w (blkcum[0] == 0).
-__device__ __forceinline__ bool locate_block(const EventSpec& ev, int w, EventBlock& eb) {
+// Inclusive scan over the wave's lanes in six DPP steps (row shifts, then the
+// row broadcasts); id is op's identity.
+template <typename Op>
+__device__ __forceinline__ int wave_scan(int x, int id, Op op) {
+  x = op(x, __builtin_amdgcn_update_dpp(id, x, 0x111, 0xf, 0xf, false));  // row_shr:1
+  x = op(x, __builtin_amdgcn_update_dpp(id, x, 0x112, 0xf, 0xf, false));
+  x = op(x, __builtin_amdgcn_update_dpp(id, x, 0x114, 0xf, 0xf, false));
+  x = op(x, __builtin_amdgcn_update_dpp(id, x, 0x118, 0xf, 0xf, false));
+  x = op(x, __builtin_amdgcn_update_dpp(id, x, 0x142, 0xa, 0xf, false));  // row_bcast:15
+  x = op(x, __builtin_amdgcn_update_dpp(id, x, 0x143, 0xc, 0xf, false));  // row_bcast:31
+  return x;
+}
+
+// The work list of a call of at most kInlineEvents events, formed by each
+// wave for itself: lane i holds event i. Sanitised token ranges, block counts
+// and the offsets' verdict are those worklist_kernel writes. A call that small
+// spent 7 us in the work-list kernel plus the launch before each direction's
+// first kernel; the wave's own list takes two loads, some forty vector
+// instructions and, for the schedules, five per event.
+constexpr int kInlineEvents = 64;
+struct InlineList {
+  int tok0, len, nblk, incl;  // this lane's event; incl: blocks of events 0 .. lane
+  bool bad;
+  __device__ __forceinline__ InlineList(const EventSpec& ev, int rows) {
+    const int lane = threadIdx.x & 63;
+    const bool in = lane < ev.B;
+    bad = false;
+    if (ev.packed) {
+      const int lo = in ? ev.lens[lane] : 0, hi = in ? ev.lens[lane + 1] : 0;
+      bad = __builtin_amdgcn_ballot_w64(in && ((lane == 0 && lo != 0) || hi < lo || (lane == ev.B - 1 && hi > ev.T))) != 0;
+      // Running maximum of the offsets, from 0, clamped to [0, T].
+      const int top = wave_scan(lo, 0, [](int a, int c) { return a > c ? a : c; });
+      tok0 = min(max(top, 0), ev.T);
+      len = in ? min(max(max(top, hi), 0), ev.T) - tok0 : 0;
+    } else {
+      const int l = in ? ev.lens[lane] : 0;
+      tok0 = 0;
+      len = l < 0 ? 0 : (l > ev.L ? ev.L : l);
+    }
+    // Padded events always get one block so that their padding rows are zeroed.
+    nblk = !in ? 0 : (len > 0 ? (len + rows - 1) / rows : (ev.packed ? 0 : 1));
+    incl = wave_scan(nblk, 0, [](int a, int c) { return a + c; });
+  }
+  // Position of this lane's event by decreasing length (ties by index), and
+  // the blocks of the events before it in that order.
+  __device__ __forceinline__ void order(int B, int& rank, int& before) const {
+    const int lane = threadIdx.x & 63;
+    rank = before = 0;
+    for (int j = 0; j < B; ++j) {
+      const int lj = __builtin_amdgcn_readlane(len, j), nj = __builtin_amdgcn_readlane(nblk, j);
+      const bool first = lj > len || (lj == len && j < lane);
+      rank += first ? 1 : 0;
+      before += first ? nj : 0;
+    }
+  }
+  // Lane b's event as eb.
+  __device__ __forceinline__ void event(int b, EventBlock& eb) const {
+    eb.b = b;
+    eb.tok0 = __builtin_amdgcn_readlane(tok0, b);
+    eb.len = __builtin_amdgcn_readlane(len, b);
+    eb.tile0 = __builtin_amdgcn_readlane(incl, b) - __builtin_amdgcn_readlane(nblk, b);
+    eb.bad = bad;
+  }
+};
+// The lane a ballot names (one bit set).
+__device__ __forceinline__ int ballot_lane(bool hit) { return __builtin_ctzll(__builtin_amdgcn_ballot_w64(hit)); }
+
+// Work item of workgroup w: the event whose blocks (of `rows` rows) hold w.
+__device__ __forceinline__ bool locate_block(const EventSpec& ev, int rows, int w, EventBlock& eb) {
+  if (ev.inl) {
+    const InlineList il(ev, rows);
+    const bool hit = w < il.incl && w >= il.incl - il.nblk;
+    if (__builtin_amdgcn_ballot_w64(hit) == 0) return false;
+    il.event(ballot_lane(hit), eb);
+    eb.blk = w - eb.tile0;
+    return true;
+  }
   if (w >= ev.blkcum[ev.B]) return false;
   const int32_t* bc = ev.blkcum;
   const int lo = wave_last_le(ev.B, w, [&](int i) { return bc[i]; });
   eb.b = lo;
-  eb.blk = w - ev.blkcum[lo];
+  eb.tile0 = ev.blkcum[lo];
+  eb.blk = w - eb.tile0;
+  eb.bad = false;
   event_range(ev, lo, eb.tok0, eb.len);
   return true;
 }

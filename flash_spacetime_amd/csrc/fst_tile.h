@@ -175,9 +175,55 @@ struct DTiles {
 // the CU's two slots between the events (cfg2 rows kernel 0.736 -> 0.713 ms;
 // the forward and cols kernel, at three per CU, keep the interleaved order,
 // which measured 1 % faster for them).
-__device__ __forceinline__ bool tile_block(const EventSpec& ev, int w, EventBlock& eb) {
+// A call without a work list (ev.inl) follows the same schedules from each
+// wave's own list; padlast stands for ev.vp there.
+__device__ __forceinline__ bool inline_tile_block(const EventSpec& ev, bool padlast, int w, EventBlock& eb) {
+  const InlineList il(ev, 16);
+  int rank, before;
+  il.order(ev.B, rank, before);
+  const int lane = threadIdx.x & 63;
+  const bool in = lane < ev.B;
+  const int x = w & 7, k = w >> 3;
   if (ev.packed) {
-    if (!ev.scum) return locate_block(ev, xcd_remap(w, gridDim.x), eb);
+    const int t = (((k >> 3) << 3) + x) * 8 + (k & 7);
+    const bool hit = in && t >= before && t < before + il.nblk;
+    if (__builtin_amdgcn_ballot_w64(hit) == 0) return false;
+    const int b = ballot_lane(hit);
+    il.event(b, eb);
+    eb.blk = t - __builtin_amdgcn_readlane(before, b);
+    return true;
+  }
+  const int nb = (ev.L + 15) >> 4;
+  // The XCD's events in order: rank 8 j + (j odd ? 7 - x : x).
+  auto nth = [&](int j) __attribute__((always_inline)) { return 8 * j + ((j & 1) ? 7 - x : x); };
+  if (!padlast) {
+    const int j = k / nb, r = nth(j);
+    if (r >= ev.B) return false;
+    il.event(ballot_lane(in && rank == r), eb);
+    eb.blk = k - j * nb;
+    return true;
+  }
+  // Valid tiles first, then the padding-only ones.
+  int rem = k;
+  for (int pass = 0; pass < 2; ++pass)
+    for (int j = 0; nth(j) < ev.B; ++j) {
+      const int b = ballot_lane(in && rank == nth(j));
+      const int v = __builtin_amdgcn_readlane(il.nblk, b), c = pass == 0 ? v : nb - v;
+      if (rem < c) {
+        il.event(b, eb);
+        eb.blk = pass == 0 ? rem : v + rem;
+        return true;
+      }
+      rem -= c;
+    }
+  return false;
+}
+
+__device__ __forceinline__ bool tile_block(const EventSpec& ev, bool padlast, int w, EventBlock& eb) {
+  if (ev.inl) return inline_tile_block(ev, padlast, w, eb);
+  eb.bad = false;
+  if (ev.packed) {
+    if (!ev.scum) return locate_block(ev, 16, xcd_remap(w, gridDim.x), eb);
     const int x = w & 7, k = w >> 3;
     const int t = (((k >> 3) << 3) + x) * 8 + (k & 7);
     if (t >= ev.scum[ev.B]) return false;
@@ -185,13 +231,14 @@ __device__ __forceinline__ bool tile_block(const EventSpec& ev, int w, EventBloc
     const int lo = wave_last_le(ev.B, t, [&](int i) { return sc[i]; });
     eb.b = ev.perm[lo];
     eb.blk = t - ev.scum[lo];
+    eb.tile0 = ev.blkcum[eb.b];
     event_range(ev, eb.b, eb.tok0, eb.len);
     return true;
   }
   const int nb = (ev.L + 15) >> 4;
   const int x = w & 7, k = w >> 3;
   int j, blk;
-  if (ev.vp) {
+  if (padlast) {
     // Padding-last: XCD x takes the valid tiles of its events (same events,
     // same order) first and their padding-only tiles after them. v[j] - v[0]
     // counts the valid tiles of the XCD's first j events, so those events'
@@ -222,6 +269,7 @@ __device__ __forceinline__ bool tile_block(const EventSpec& ev, int w, EventBloc
   const int b = ev.perm[r];
   eb.b = b;
   eb.blk = blk;
+  eb.tile0 = ev.blkcum[b];
   event_range(ev, b, eb.tok0, eb.len);
   return true;
 }
