@@ -124,6 +124,25 @@ def load() -> ctypes.CDLL:
     return _LIB
 
 
+_HOST = None
+
+
+def host():
+    """The host extension (csrc/fst_host.cpp), bound once to the loaded library."""
+    global _HOST
+    if _HOST is None:
+        lib = load()
+        try:
+            from . import _fst_host
+        except ImportError as e:
+            raise LibraryMissing(f"{e}: build it with `python -m flash_spacetime_amd.build`") from e
+        _fst_host.bind_library(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in (
+            "fst_supported", "fst_forward_workspace_bytes", "fst_forward", "fst_backward_workspace_bytes",
+            "fst_backward")))
+        _HOST = _fst_host
+    return _HOST
+
+
 def last_error() -> str:
     return load().fst_last_error().decode()
 

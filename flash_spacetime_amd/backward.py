@@ -17,11 +17,21 @@ import torch
 from torch import Tensor
 
 from . import _lib, tune
-from .forward import _Prepared, _bf16, _vec_in_layout, head_groups
+from .forward import _Prepared, _bf16, _raw_stream, _vec_in_layout, head_groups
 
 
 def _same_layout(a: Tensor, b: Tensor) -> bool:
     return all(sa == sb for sa, sb, n in zip(a.stride(), b.stride(), a.shape) if n > 1)
+
+
+def _native_backward(dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, scale, out=None):
+    """The backward through the host extension: (dq, dk, dv, dw, db), or for an
+    interleaved q (k and v None) (dqkv, None, None, dw, db); None where the call is
+    not in the form it takes or runs another than the static plan, for
+    `_run_backward` to run or reject."""
+    if not (q.is_cuda and tune.static_only()):
+        return None
+    return _lib.host().backward(dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, scale, out, _raw_stream(q))
 
 
 def _run_backward(dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, scale, vec_shape,

@@ -1,4 +1,5 @@
-"""Build the gfx950 HIP library `libflash_spacetime.so` in the package directory.
+"""Build the gfx950 HIP library `libflash_spacetime.so` and the host extension
+`_fst_host.so` in the package directory.
 
 Every kernel instance family is its own translation unit so hipcc runs them
 in parallel; the objects are linked into one shared library whose C ABI is
@@ -20,6 +21,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 BUILD = CSRC / "_build"
 LIB = PKG / "libflash_spacetime.so"
+HOST_LIB = PKG / "_fst_host.so"
 
 ARCH = os.environ.get("FST_OFFLOAD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
@@ -72,6 +74,27 @@ def _units():
     return [u for u in units if u[1].exists()]
 
 
+def _build_host():
+    """Compile csrc/fst_host.cpp, the operators' host path (a Python extension
+    against torch's C++ API; no device code)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    tmp = HOST_LIB.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+           "-DTORCH_EXTENSION_NAME=_fst_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}"]
+    for inc in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"]):
+        cmd += ["-isystem", str(inc)]
+    cmd += [str(CSRC / "fst_host.cpp"), "-o", str(tmp)]
+    cmd += [f"-L{p}" for p in cpp_extension.library_paths()] + ["-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("host extension failed:\n" + res.stdout + res.stderr)
+    os.replace(tmp, HOST_LIB)
+
+
 RESOURCES = BUILD / "kernel_resources.json"
 _REMARK = re.compile(r"remark:\s+(Function Name|VGPRs|AGPRs|ScratchSize \[bytes/lane\]|Occupancy \[waves/SIMD\]"
                      r"|LDS Size \[bytes/block\]): (\S+)")
@@ -114,7 +137,9 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
     units = _units()
     jobs = jobs or min(len(units), max(1, min(16, os.cpu_count() or 1)))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_build_host)
         results = list(pool.map(_compile, units))
+        host.result()
     failed = [r for r in results if r[2] != 0]
     for name, _, rc, out, _ in results:
         if out.strip() and (verbose or rc != 0):

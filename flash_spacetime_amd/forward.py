@@ -256,6 +256,33 @@ class _Prepared:
         return torch.empty(self.vec_shape(), device=self.device, dtype=torch.float32)
 
 
+_PLAIN = (Tensor, torch.nn.Parameter)
+
+
+def _native_forward(q, k, v, feats, weight, bias, lens, scale, use_attn_bias, use_activation_bias, packed,
+                    interleaved=False):
+    """The forward through the host extension, or None where the call is not in
+    the form it takes (csrc/fst_host.cpp) or a plan other than the static one
+    is asked for; the Python path below then runs or rejects it. interleaved: q
+    is one contiguous interleaved tensor, k and v are None. Returns (out, lse, q, k, v, pos4,
+    weight, bias, lens, dims, scale) as `_Prepared` and `_run_forward` form them."""
+    if not (q.is_cuda and tune.static_only() and (scale is None or type(scale) in (float, int))
+            and (k is None) == interleaved and (v is None) == interleaved):
+        return None
+    # Tensor subclasses keep their own methods: the Python path calls them.
+    for t in (q, feats, weight, lens) if interleaved else (q, k, v, feats, weight, lens):
+        if type(t) not in _PLAIN:
+            return None
+    if bias is not None and type(bias) not in _PLAIN:
+        return None
+    return _lib.host().forward(q, k, v, feats, weight, bias, lens, scale, bool(use_attn_bias),
+                               bool(use_activation_bias), packed, _raw_stream(q))
+
+
+def _raw_stream(t: Tensor) -> int:
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
 def _run_forward(prep: _Prepared) -> Tuple[Tensor, Tensor]:
     lib = _lib.load()
     out = prep.empty_out()
@@ -283,6 +310,18 @@ def _run_forward(prep: _Prepared) -> Tuple[Tensor, Tensor]:
         rc = run(dims[1] | plan)
     _lib.check(rc, "flash_spacetime_forward")
     return out, lse
+
+
+def _python_forward(prep: _Prepared):
+    """_native_forward's result from the Python path."""
+    out, lse = _run_forward(prep)
+    return (out, lse, prep.q, prep.k, prep.v, prep.pos4, prep.weight, prep.bias, prep.lens, prep.dims(), prep.scale)
+
+
+def vec_shape(dims: Tuple[int, ...]) -> Tuple[int, ...]:
+    """Shape of the per-row vectors (lse, rowsum) of a call's dims."""
+    _, flags, batch, heads, length, tokens, _, _ = dims
+    return (tokens, heads) if flags & _lib.FST_PACKED else (batch, heads, length)
 
 
 def flash_spacetime_forward(
@@ -325,10 +364,14 @@ def flash_spacetime_forward(
                                            use_activation_bias, block_m=block_m, block_n=block_n,
                                            num_warps=num_warps, cu_seqlens=cu_seqlens)
         return out.to(_HALF), lse
-    prep = _Prepared(q, k, v, feats, weight, bias, seqlens, scale, use_attn_bias,
-                     use_activation_bias, cu_seqlens)
     with tune.tile_request(block_m, block_n, None):
-        return _run_forward(prep)
+        packed = cu_seqlens is not None
+        done = _native_forward(q, k, v, feats, weight, bias, cu_seqlens if packed else seqlens, scale, use_attn_bias,
+                               use_activation_bias, packed)
+        if done is not None:
+            return done[0], done[1]
+        return _run_forward(_Prepared(q, k, v, feats, weight, bias, seqlens, scale, use_attn_bias,
+                                      use_activation_bias, cu_seqlens))
 
 
 _TEMPORARY_OUTPUT = threading.local()
@@ -401,19 +444,18 @@ class _FlashSpacetimeAttention(torch.autograd.Function):
     ) -> Tensor:
         if feats.requires_grad:
             raise ValueError("feats (detector data) must not require grad")
-        prep = _Prepared(q, k, v, feats, weight, bias, seqlens, scale, use_attn_bias,
-                         use_activation_bias, cu_seqlens)
-        out, lse = _run_forward(prep)
+        packed = cu_seqlens is not None
+        done = _native_forward(q, k, v, feats, weight, bias, cu_seqlens if packed else seqlens, scale, use_attn_bias,
+                               use_activation_bias, packed)
+        if done is None:
+            done = _python_forward(_Prepared(q, k, v, feats, weight, bias, seqlens, scale, use_attn_bias,
+                                             use_activation_bias, cu_seqlens))
+        out, lse, qc, kc, vc, pos4, w32, b32, lens, ctx.dims, ctx.scale = done
         # The inputs and the LSE are saved as the reference saves them
         # (forward.py:381-388); the backward forms its own softmax row sums.
-        ctx.save_for_backward(prep.q, prep.k, prep.v, prep.pos4, prep.lens, lse, *_keep_output(ctx, out))
-        ctx.prep_meta = (prep.weight, prep.bias, weight.dtype,
-                         None if bias is None else bias.dtype)
-        ctx.dims = prep.dims()
-        ctx.scale = prep.scale
-        ctx.packed = prep.packed
+        ctx.save_for_backward(qc, kc, vc, pos4, lens, lse, *_keep_output(ctx, out))
+        ctx.prep_meta = (w32, b32, weight.dtype, None if bias is None else bias.dtype)
         ctx.flags = (use_attn_bias, use_activation_bias)
-        ctx.vec_shape = prep.vec_shape()
         return out
 
     @staticmethod
@@ -423,14 +465,16 @@ class _FlashSpacetimeAttention(torch.autograd.Function):
                 "FLASH_ST_REFERENCE_BWD=1 (autograd through the materialised reference) is not "
                 "offered: this build has only the fused HIP backward"
             )
-        from .backward import _run_backward
+        from .backward import _native_backward, _run_backward
 
         q, k, v, pos4, lens, lse, *kept = ctx.saved_tensors
         w32, b32, w_dtype, b_dtype = ctx.prep_meta
-        dq, dk, dv, dw, db = _run_backward(
-            ctx.dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, ctx.scale, ctx.vec_shape,
-            out=_kept_output(ctx, kept),
-        )
+        out = _kept_output(ctx, kept)
+        grads = _native_backward(ctx.dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, ctx.scale, out)
+        if grads is None:
+            grads = _run_backward(ctx.dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, ctx.scale,
+                                  vec_shape(ctx.dims), out=out)
+        dq, dk, dv, dw, db = grads
         use_attn_bias, use_activation_bias = ctx.flags
         proj_used = use_attn_bias or use_activation_bias
         w_needed, b_needed = ctx.needs_input_grad[4], ctx.needs_input_grad[5]
@@ -595,38 +639,43 @@ class _FlashSpacetimeAttentionQKV(torch.autograd.Function):
         if feats.requires_grad:
             raise ValueError("feats (detector data) must not require grad")
         packed = cu_seqlens is not None
-        q, k, v = _qkv_views(qkv, packed)
-        prep = _Prepared(q, k, v, feats, weight, bias, seqlens, scale, use_attn_bias,
-                         use_activation_bias, cu_seqlens, interleaved=True)
-        out, lse = _run_forward(prep)
+        done = _native_forward(qkv, None, None, feats, weight, bias, cu_seqlens if packed else seqlens, scale,
+                               use_attn_bias, use_activation_bias, packed, interleaved=True)
+        if done is None:
+            q, k, v = _qkv_views(qkv, packed)
+            done = _python_forward(_Prepared(q, k, v, feats, weight, bias, seqlens, scale, use_attn_bias,
+                                             use_activation_bias, cu_seqlens, interleaved=True))
+        out, lse, _, _, _, pos4, w32, b32, lens, ctx.dims, ctx.scale = done
         ret = out if packed else out.transpose(1, 2)  # [T, H, D] / [B, L, H, D], dense
-        ctx.save_for_backward(qkv, prep.pos4, prep.lens, lse, *_keep_output(ctx, out, ret))
-        ctx.prep_meta = (prep.weight, prep.bias, weight.dtype, None if bias is None else bias.dtype)
-        ctx.dims = prep.dims()
-        ctx.scale = prep.scale
+        ctx.save_for_backward(qkv, pos4, lens, lse, *_keep_output(ctx, out, ret))
+        ctx.prep_meta = (w32, b32, weight.dtype, None if bias is None else bias.dtype)
         ctx.packed = packed
         ctx.flags = (use_attn_bias, use_activation_bias)
-        ctx.vec_shape = prep.vec_shape()
         return ret
 
     @staticmethod
     def backward(ctx: Any, grad_out: Tensor) -> Tuple[Optional[Tensor], ...]:  # type: ignore[override]
-        from .backward import _run_backward
+        from .backward import _native_backward, _run_backward
 
         qkv, pos4, lens, lse, *kept = ctx.saved_tensors
         w32, b32, w_dtype, b_dtype = ctx.prep_meta
-        q, k, v = _qkv_views(qkv, ctx.packed)
-        dqkv = torch.empty_like(qkv)
         g = grad_out if ctx.packed else grad_out.transpose(1, 2)
-        if ctx.packed:
-            like = torch.empty(q.shape, device=qkv.device, dtype=qkv.dtype)
+        out = _kept_output(ctx, kept)
+        grads = _native_backward(ctx.dims, qkv, None, None, pos4, w32, b32, lens, lse, g, ctx.scale, out)
+        if grads is not None:
+            dqkv, _, _, dw, db = grads
         else:
-            b, h, length, d = q.shape
-            like = torch.empty(b, length, h, d, device=qkv.device, dtype=qkv.dtype).transpose(1, 2)
-        _, _, _, dw, db = _run_backward(
-            ctx.dims, q, k, v, pos4, w32, b32, lens, lse, g, ctx.scale, ctx.vec_shape,
-            out_like=like, grads=_qkv_views(dqkv, ctx.packed), out=_kept_output(ctx, kept),
-        )
+            q, k, v = _qkv_views(qkv, ctx.packed)
+            dqkv = torch.empty_like(qkv)
+            if ctx.packed:
+                like = torch.empty(q.shape, device=qkv.device, dtype=qkv.dtype)
+            else:
+                b, h, length, d = q.shape
+                like = torch.empty(b, length, h, d, device=qkv.device, dtype=qkv.dtype).transpose(1, 2)
+            _, _, _, dw, db = _run_backward(
+                ctx.dims, q, k, v, pos4, w32, b32, lens, lse, g, ctx.scale, vec_shape(ctx.dims),
+                out_like=like, grads=_qkv_views(dqkv, ctx.packed), out=out,
+            )
         use_attn_bias, use_activation_bias = ctx.flags
         proj_used = use_attn_bias or use_activation_bias
         return (

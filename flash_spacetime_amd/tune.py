@@ -133,6 +133,12 @@ def tile_request(block_m: Optional[int] = None, block_n: Optional[int] = None, n
         _tiles.reset(token)
 
 
+def static_only() -> bool:
+    """Whether a call now runs the library's static plan, whatever its shape:
+    no tuner, no fixed plan, no tile arguments."""
+    return not _enabled and _fixed is None and _tiles.get() is None
+
+
 def _tiled(kind: str, dims: Tuple[int, ...]) -> Optional[int]:
     req = _tiles.get()
     return None if req is None else plan_from_tiles(dims[0], dims[3], dims[6], dims[7], kind, *req)

@@ -17,7 +17,7 @@ ROOT = Path(__file__).resolve().parent
 
 
 class BuildWithKernels(build_py):
-    """Compile libflash_spacetime.so before the package files are copied."""
+    """Compile libflash_spacetime.so and _fst_host.so before the package files are copied."""
 
     def run(self):
         spec = importlib.util.spec_from_file_location("fst_build", ROOT / "flash_spacetime_amd" / "build.py")
@@ -38,7 +38,7 @@ setup(
     install_requires=["torch>=2.4"],
     extras_require={"dev": ["pytest>=7"]},
     packages=["flash_spacetime_amd"],
-    package_data={"flash_spacetime_amd": ["libflash_spacetime.so"]},
+    package_data={"flash_spacetime_amd": ["libflash_spacetime.so", "_fst_host.so"]},
     cmdclass={"build_py": BuildWithKernels},
     zip_safe=False,
 )
