@@ -63,7 +63,8 @@ __device__ __forceinline__ void finish_p_dp(f32x4& s, f32x4& dp, float lse2, flo
 template <typename T, int HP, int D, int C, int NW, int NS>
 struct BwdRowsCfg {
   static constexpr bool BF = is_bf16<T>::value;
-  static constexpr int HW = HP / NW, RW = 16 / NW;
+  using HS = HeadSplit<HP, NW>;
+  static constexpr int HW = HS::HW, RW = 16 / NW;
   static constexpr int WPG = NW > 4 ? NW : 4, THREADS = 64 * WPG;  // waves, threads per workgroup
   static constexpr int TILES = WPG / NW, ROWS = 16 * TILES;
   static constexpr int KC = 16 * NS;
@@ -128,7 +129,7 @@ struct BwdRowsCfg {
   // A row-owner wave's RW rows x KC keys: whole embeddings per lane, or
   // whole groups of four frequencies per lane where lanes share a pair.
   using EL = EmbedLanes<RW * KC>;
-  static constexpr bool FITS = LDS_BYTES <= 160 * 1024 && HP % NW == 0 && EL::OK && (C / 2 / EL::SPLIT) % 4 == 0;
+  static constexpr bool FITS = LDS_BYTES <= 160 * 1024 && HS::OK && EL::OK && (C / 2 / EL::SPLIT) % 4 == 0;
   static_assert(SLOT % 16 == 0, "slot alignment");
 };
 
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_rows_kernel(Bwd
   float lse2[HW], dobv[HW], nsum[HW], zsum[HW], dval[HW], sig[HW], zlane[HW];
 #pragma unroll
   for (int hl = 0; hl < HW; ++hl) {
-    const int h = ws * HW + hl;
+    const int h = Cfg::HS::head(ws, hl);
     const bool ok = h < H && row_ok;
     if (ok) {
       qf[hl].load_scaled(qg + rx.off(h, my_row, D), g, prm.scale);
@@ -342,7 +343,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_rows_kernel(Bwd
       if constexpr (KE) {
 #pragma unroll
         for (int hl = 0; hl < HW; ++hl) {
-          const int hc = min(ws * HW + hl, H - 1);
+          const int hc = min(Cfg::HS::head(ws, hl), H - 1);
 #pragma unroll
           for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
@@ -390,7 +391,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_rows_kernel(Bwd
       // ---- head-owner: P, dP, online D, dS, dQ ----
 #pragma unroll
       for (int hl = 0; hl < HW; ++hl) {
-        const int h = ws * HW + hl;
+        const int h = Cfg::HS::head(ws, hl);
         if (h >= H) continue;
         f32x4 S[NS], P_[NS];
         const float* slot = Sf + (n * HP + h) * SLOT_F;
@@ -533,7 +534,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_rows_kernel(Bwd
   float rz[HW];
 #pragma unroll
   for (int hl = 0; hl < HW; ++hl) {
-    const int h = ws * HW + hl;
+    const int h = Cfg::HS::head(ws, hl);
     rz[hl] = zsum[hl] > 0.f ? 1.f / zsum[hl] : 1.f;
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt) dQ[hl][dt] = dQ[hl][dt] * rz[hl];
@@ -541,7 +542,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_rows_kernel(Bwd
       prm.dsum[ra.vec(h, my_row)] = dval[hl];
       prm.lse_z[ra.vec(h, my_row)] = zsum[hl] > 0.f ? log2f(zsum[hl]) : 0.f;
     }
-    if (use_e && g == 0) Dd[h * 16 + n] = rz[hl];
+    if (use_e && g == 0 && h < HP) Dd[h * 16 + n] = rz[hl];
   }
   if (use_e) {
     __syncthreads();
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_rows_kernel(Bwd
 #pragma unroll
   for (int hl = 0; hl < HW; ++hl) {
     sig[hl] = group_allsum(sig[hl]) * rz[hl];
-    const int h = ws * HW + hl;
+    const int h = Cfg::HS::head(ws, hl);
     if (prm.rowsum && g == 0 && h < H && row_ok) prm.rowsum[ra.vec(h, my_row)] = sig[hl];
   }
   T* dqg = reinterpret_cast<T*>(prm.dq);
@@ -582,7 +583,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_rows_kernel(Bwd
     }
 #pragma unroll
     for (int hl = 0; hl < HW; ++hl) {
-      const int h = ws * HW + hl;
+      const int h = Cfg::HS::head(ws, hl);
       if (h >= H) continue;
       f32x4 o = dQ[hl][dt];
       if (attn) {
@@ -691,7 +692,8 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_rows_kernel(Bwd
 template <typename T, int HP, int D, int C, int NW, int NS>
 struct BwdColsCfg {
   static constexpr bool BF = is_bf16<T>::value;
-  static constexpr int HW = HP / NW;
+  using HS = HeadSplit<HP, NW>;
+  static constexpr int HW = HS::HW;
   static constexpr int WPG = NW > 4 ? NW : 4, THREADS = 64 * WPG;  // waves, threads per workgroup
   static constexpr int TILES = WPG / NW, KEYS = 16 * TILES;
   static constexpr int KC = 16 * NS;          // streamed rows per chunk
@@ -728,7 +730,7 @@ struct BwdColsCfg {
   // whole groups of four frequencies per lane where lanes share a pair.
   using EL = EmbedLanes<RWS * 16>;
   static constexpr bool FITS =
-      LDS_BYTES <= 160 * 1024 && HP % NW == 0 && RWS >= 1 && EL::OK && (C / 2 / EL::SPLIT) % 4 == 0;
+      LDS_BYTES <= 160 * 1024 && HS::OK && RWS >= 1 && EL::OK && (C / 2 / EL::SPLIT) % 4 == 0;
 };
 
 template <typename T, int HP, int D, int C, int NW, int NS>
@@ -784,7 +786,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_cols_kernel(Bwd
   f32x4 dK[HW][D / 16], dV[HW][D / 16];
 #pragma unroll
   for (int hl = 0; hl < HW; ++hl) {
-    const int h = ws * HW + hl;
+    const int h = Cfg::HS::head(ws, hl);
     if (h < H && key_ok) {
       kf[hl].load(kg + rx.off(h, my_key, D), g);
       vf[hl].load(vg + rx.off(h, my_key, D), g);
@@ -1025,7 +1027,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_cols_kernel(Bwd
     // ---- head-owner: S = qt k^T + u.E, P, dP, dS; dv += dO^T P, dk += qt^T dS ----
 #pragma unroll
     for (int hl = 0; hl < HW; ++hl) {
-      const int h = ws * HW + hl;
+      const int h = Cfg::HS::head(ws, hl);
       if (h >= H) continue;
       f32x4 S[NS], dP[NS], dS[NS];
 #pragma unroll
@@ -1098,7 +1100,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_cols_kernel(Bwd
   T* dvg = reinterpret_cast<T*>(prm.dv);
 #pragma unroll
   for (int hl = 0; hl < HW; ++hl) {
-    const int h = ws * HW + hl;
+    const int h = Cfg::HS::head(ws, hl);
     if (h >= H || !key_ok) continue;
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt) {
@@ -1140,7 +1142,7 @@ struct BwdPick {
 // took 22.7 ms against 31.7 for two.
 template <int HP, int D, int C, int NW>
 constexpr int rows_static_passes() {
-  return (HP / NW) * D + (16 / NW) * C <= 256 ? 1 : 2;
+  return HeadSplit<HP, NW>::HW * D + (16 / NW) * C <= 256 ? 1 : 2;
 }
 
 template <typename T, int HP, int D, int C, int NW, int NS>
@@ -1200,7 +1202,11 @@ int bwd_launch_t(const BwdParams& prm, int which, hipStream_t stream, int grid, 
   if constexpr (!PR::OK || !PC::OK) {
     return FST_EUNSUPPORTED;
   } else {
-    const int nw = plan_nw(prm.flags, bit_index(FST_PLAN_BWD_T16), bit_index(FST_PLAN_BWD_W8));
+    int nw = plan_nw(prm.flags, bit_index(FST_PLAN_BWD_T16), bit_index(FST_PLAN_BWD_W8));
+    // Two shapes of 12 heads where the eight-wave kernel spills and four waves
+    // are no slower (B = 24, L = 768: D = 64, C = 48 rows 2.21 against 2.31 ms;
+    // D = 64, C = 16 cols 1.34 against 1.32, B = 32 1.69 against 1.74).
+    if (nw == 0 && HP == 12 && D == 64 && C == (which == 0 ? 48 : 16)) nw = 4;
     const int ns = plan_ns(prm.flags, bit_index(FST_PLAN_BWD_KC16));
     const int split = which == 0 ? pick_split<PR::template F>(nw, ns, 1) : pick_split<PC::template F>(nw, ns, 1);
     switch (split) {

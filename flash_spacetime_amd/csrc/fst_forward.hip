@@ -35,7 +35,8 @@ namespace fst {
 template <typename T, int HP, int D, int C, int NW, int NS>
 struct FwdCfg {
   static constexpr bool BF = is_bf16<T>::value;
-  static constexpr int HW = HP / NW;     // heads per head-owner wave
+  using HS = HeadSplit<HP, NW>;
+  static constexpr int HW = HS::HW;      // heads per head-owner wave (at most)
   static constexpr int RW = 16 / NW;     // rows per row-owner wave
   static constexpr int WPG = NW > 4 ? NW : 4;  // waves per workgroup
   static constexpr int THREADS = 64 * WPG;
@@ -77,7 +78,7 @@ struct FwdCfg {
   // A row-owner wave's RW rows x KC keys: whole embeddings per lane, or
   // whole groups of four frequencies per lane where lanes share a pair.
   using EL = EmbedLanes<RW * KC>;
-  static constexpr bool FITS = LDS_BYTES <= 160 * 1024 && HP % NW == 0 && EL::OK && (C / 2 / EL::SPLIT) % 4 == 0 &&
+  static constexpr bool FITS = LDS_BYTES <= 160 * 1024 && HS::OK && EL::OK && (C / 2 / EL::SPLIT) % 4 == 0 &&
                                !(BF && NS != 1 && NS != 2);
   static_assert(SLOT % 16 == 0, "slots must stay 16-byte aligned");
 };
@@ -134,7 +135,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void fwd_kernel(FwdParam
   float m_run[HW], l_run[HW];
 #pragma unroll
   for (int hl = 0; hl < HW; ++hl) {
-    const int h = ws * HW + hl;
+    const int h = Cfg::HS::head(ws, hl);
     if (h < H && row_ok)
       qf[hl].load_scaled(qg + rx.off(h, my_row, D), g, prm.scale);
     else
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void fwd_kernel(FwdParam
     // ---- head-owner: logits, online softmax, P V ----
 #pragma unroll
     for (int hl = 0; hl < HW; ++hl) {
-      const int h = ws * HW + hl;
+      const int h = Cfg::HS::head(ws, hl);
       if (h >= H) continue;
       // VE: this head's V columns (gathered element by element from clamped
       // keys, zeroed past the event) are loaded before its logits, so they
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void fwd_kernel(FwdParam
   for (int hl = 0; hl < HW; ++hl) {
     const float lf = group_allsum(l_run[hl]);
     inv_l[hl] = 1.f / lf;
-    const int h = ws * HW + hl;
+    const int h = Cfg::HS::head(ws, hl);
     if (g == 0 && row_ok && h < H) prm.lse[ra.vec(h, my_row)] = m_run[hl] + logf(lf);
   }
 
@@ -374,7 +375,7 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void fwd_kernel(FwdParam
     }
 #pragma unroll
     for (int hl = 0; hl < HW; ++hl) {
-      const int h = ws * HW + hl;
+      const int h = Cfg::HS::head(ws, hl);
       if (h >= H) continue;
       f32x4 o = O[hl][dt];
       if (act) o = o + *reinterpret_cast<const f32x4*>(Sf + (n * HP + h) * SLOT_F + 4 * g);
@@ -406,12 +407,15 @@ struct FwdPick {
   template <int NW, int NS>
   using F = FwdCfg<T, HP, D, C, NW, NS>;
   // The split for requested (nw, ns) (0: not requested). An eight-wave tile
-  // whose waves own two heads or more takes 16-key chunks first (H = 16,
-  // D = 32, C = 16, B = 64, L = 768: 0.83 against 1.08 ms; with one head per
-  // wave 32-key chunks stay first: cfg4 11.2 against 15.1 ms).
+  // whose waves own two heads takes 16-key chunks first at C = 16 (H = 16,
+  // D = 32, B = 64, L = 768: 0.83 against 1.08 ms; H = 12, B = 24: 0.316 against
+  // 0.378); with more channels, or one head per wave, 32-key chunks stay first
+  // (B = 24, L = 768: H = 12, D = C = 32 0.371 against 0.460, D = 48, C = 48
+  // 0.543 against 0.674, H = 16, D = C = 32 0.421 against 0.516; H = 8,
+  // D = C = 64, B = 8, L = 4096: 11.2 against 15.1 ms).
   static constexpr int choose(int nw, int ns) {
     const int s = pick_split<F>(nw, ns);
-    return ns == 0 && s / 10 == 8 && HP / 8 >= 2 ? pick_split<F>(8, 0, 1) : s;
+    return ns == 0 && s / 10 == 8 && F<8, 1>::HW >= 2 && C == 16 ? pick_split<F>(nw, 0, 1) : s;
   }
   static constexpr int STATIC = choose(0, 0);
   static constexpr int NW = STATIC ? STATIC / 10 : 4, NS = STATIC ? STATIC % 10 : 1;

@@ -588,6 +588,9 @@ constexpr int pick_split(int nw, int ns, int ns_first = 2) {
   const int nws[4] = {8, 4, 2, 1};
   for (int w = 0; w < 4; ++w) {
     if (nw && nws[w] != nw) continue;
+    // The eight-wave plan bits stand for even splits; the uneven one is a
+    // static choice only.
+    if (nw == 8 && !F<8, 1>::HS::EVEN) continue;
     for (int k = 0; k < 2; ++k) {
       const int s = k == 0 ? ns_first : 3 - ns_first;
       if (ns && s != ns) continue;
@@ -607,6 +610,25 @@ __host__ __device__ inline int plan_nw(int flags, int t, int w8) {
 }
 __host__ __device__ inline int plan_ns(int flags, int k) { return (flags >> k) & 1 ? 1 : ((flags >> (k + 1)) & 1 ? 2 : 0); }
 constexpr int bit_index(int b) { return b <= 1 ? 0 : 1 + bit_index(b >> 1); }
+
+// Heads of a 16-row tile's NW waves: ceil(HP / NW) a wave, one fewer from wave
+// NBIG on where NW does not divide HP (eight waves of 12 heads: 2 and 1; waves
+// w and w + 4 share a SIMD, so every SIMD serves three). Twelve heads over four
+// waves kept the float32 kernels at one wave per SIMD (311 to 411 registers a
+// lane at D = 32, C = 16); over eight they run two: H = 12, D = 32, C = 16, B = 32,
+// L = 768, lengths U{16..768}: forward 0.457 -> 0.414 ms, rows 0.795 -> 0.638,
+// cols 1.004 -> 0.683; the other widths -14 to -41 % (rows), -23 to -32 % (cols).
+template <int HP, int NW>
+struct HeadSplit {
+  static constexpr int HW = (HP + NW - 1) / NW, NBIG = HP - NW * (HW - 1);
+  static constexpr bool EVEN = HP % NW == 0, OK = EVEN || (NW == 8 && HP == 12);
+  // Head hl of wave ws, or one past every head.
+  static __device__ __forceinline__ int head(int ws, int hl) {
+    if constexpr (EVEN) return ws * HW + hl;
+    if (ws < NBIG) return ws * HW + hl;
+    return hl < HW - 1 ? NBIG * HW + (ws - NBIG) * (HW - 1) + hl : HP;
+  }
+};
 
 // The plan bits of a (NW, NS) family: a tile-height bit for each NW and a
 // key-chunk bit for each NS that fits with some value of the other.
