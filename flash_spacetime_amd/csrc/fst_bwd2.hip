@@ -1380,6 +1380,12 @@ struct Bwd2Pick {
   // against 0.437 ms; within 1 % elsewhere).
   static constexpr int ROWS_STATIC = NW == 8 ? 2 : ((HP % 8 == 0 && ROWS_W8X2) ? 3 : 1);
   static constexpr int COLS_STATIC = COLS_OCC3 ? 3 : 2;
+  // Twelve heads of a heavy lane state run the rows kernel's eight waves, one
+  // workgroup per CU, unpadded: two heads on waves 0 to 3, one on the others
+  // (three a SIMD), where padding to 16 gave every SIMD four: B = 64, L = 768,
+  // lengths U{16..768}: D = C = 32 0.320 -> 0.306 ms, D = C = 64 1.536 -> 1.368,
+  // D = 64, C = 48 -6 %, the other widths 0 to -4 % (bit for bit the same).
+  static constexpr bool ROWS_U8 = HP == 12 && !LIGHT && Rows2Cfg<HP, D, C, KC, 8>::FITS;
   // Eight cols-kernel waves per workgroup, each with half the heads of a
   // four-wave one and two rows of each chunk (the same arithmetic), as waves
   // per SIMD; 0: COLS_STATIC. At HP = 16 the four-wave instances spill from
@@ -1461,6 +1467,9 @@ static int bwd2_launch_t(const BwdParams& prm, int which, hipStream_t stream, in
     return FST_EUNSUPPORTED;
 #else
     const bool kl = f & FST_PLAN_ROWS_KV_LDS;
+    if constexpr (P::ROWS_U8)
+      if (!kl && !(f & (FST_PLAN_ROWS_W4 | FST_PLAN_ROWS_W8 | FST_PLAN_ROWS_W8X2)))
+        return bwd2_launch_rows<HP, D, C, 8, 2, false>(prm, stream, g8, query);
     const int waves = (f & FST_PLAN_ROWS_W4)     ? 1
                       : (f & FST_PLAN_ROWS_W8)   ? 2
                       : (f & FST_PLAN_ROWS_W8X2) ? 3

@@ -29,21 +29,21 @@ static bool supported_dim(int x) { return x == 16 || x == 32 || x == 48 || x == 
 
 static int head_padding(int H) { return H <= 4 ? 4 : (H <= 8 ? 8 : (H <= 12 ? 12 : 16)); }
 
-// Head padding of the bf16 rows kernel: where its four-wave instance would
-// spill, heads are padded to the next multiple of 8 so that it runs eight
-// waves (padded heads compute on a real head's data and store nothing). The
-// scratch between the rows and cols kernel is laid out by H, so each pads as
-// it likes.
-// The eight-wave, one-workgroup plan (FST_PLAN_ROWS_W8) pads to a multiple
-// of 8 likewise; the four-wave plan and the eight-wave, two-workgroup plan
-// (which gives waves 4 to 7 one head fewer where 8 does not divide the
-// padding) keep head_padding.
+// Head padding of the bf16 rows kernel: up to four heads are padded to 8 where
+// the four-wave instance would spill, so that it runs eight waves (padded
+// heads compute on a real head's data and store nothing; 12 heads split over
+// eight waves unpadded). The scratch between the rows and cols kernel is laid
+// out by H, so each pads as it likes.
+// The eight-wave, one-workgroup plan (FST_PLAN_ROWS_W8) pads to a multiple of
+// 8; the four-wave plan and the eight-wave, two-workgroup plan (which gives
+// waves 4 to 7 one head fewer where 8 does not divide the padding) keep
+// head_padding.
 static int rows_head_padding(int dtype, int flags, int H, int D, int C) {
   const int hp = head_padding(H);
   if (dtype != FST_BF16) return hp;
   if (flags & FST_PLAN_ROWS_W8) return (hp + 7) & ~7;
   if (flags & (FST_PLAN_ROWS_W4 | FST_PLAN_ROWS_W8X2)) return hp;
-  if (hp % 8 != 0 && rows_wave_load(hp, D, C) >= 160) return hp + 4;
+  if (hp == 4 && rows_wave_load(hp, D, C) >= 160) return 8;
   return hp;
 }
 
