@@ -746,10 +746,14 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_cols_kernel(Bwd
   const int wave = tid >> 6, lane = tid & 63, g = lane >> 4, n = lane & 15;
   const int tile = wave / NW, ws = wave % NW;
 
+  if ((int)blockIdx.x < prm.red_blocks) {
+    reduce_block<D * C, D>(prm, tid, reinterpret_cast<float*>(smem));
+    return;
+  }
   EventSpec ev = prm.ev;
   ev.blkcum = prm.blkcum_cols;
   EventBlock eb;
-  if (!locate_block(ev, Cfg::KEYS, blockIdx.x, eb)) return;
+  if (!locate_block(ev, Cfg::KEYS, blockIdx.x - prm.red_blocks, eb)) return;
   const int len = eb.len;
   const int H = prm.H;
   const bool attn = prm.flags & FST_ATTN_BIAS;
@@ -1175,7 +1179,8 @@ int bwd_launch_v(const BwdParams& prm, int which, hipStream_t stream, int grid, 
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, K::LDS_BYTES) !=
         hipSuccess)
       return FST_ELAUNCH;
-    if (grid > 0) hipLaunchKernelGGL(kern, dim3(grid), dim3(K::THREADS), K::LDS_BYTES, stream, prm);
+    if (grid > 0)
+      hipLaunchKernelGGL(kern, dim3(grid + prm.red_blocks), dim3(K::THREADS), K::LDS_BYTES, stream, prm);
     return hipGetLastError() == hipSuccess ? FST_OK : FST_ELAUNCH;
   }
 }

@@ -938,12 +938,16 @@ __global__ __launch_bounds__(64 * NW, OCC) void bwd_cols2_kernel(BwdParams prm) 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
 
+  if ((int)blockIdx.x < prm.red_blocks) {
+    reduce_block<D * C, D>(prm, tid, reinterpret_cast<float*>(smem));
+    return;
+  }
   EventSpec ev = prm.ev;
   ev.blkcum = prm.blkcum_cols;
   ev.scum = prm.scum_cols;
   EventBlock eb;
   // The interleaved schedule (the padding-last one is the rows kernel's).
-  if (!tile_block(ev, false, blockIdx.x, eb)) return;
+  if (!tile_block(ev, false, blockIdx.x - prm.red_blocks, eb)) return;
   const int len = eb.len;
   const int H = prm.H;
   // FL >= 0: the bias flags fixed at compile time; -1: read at run time.
@@ -1440,7 +1444,8 @@ int bwd2_launch_cols(const BwdParams& prm, hipStream_t stream, int g8, bool quer
   if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES) !=
       hipSuccess)
     return FST_ELAUNCH;
-  if (g8 > 0) hipLaunchKernelGGL(kern, dim3(g8), dim3(64 * NW), Cfg::LDS_BYTES, stream, prm);
+  if (g8 > 0)
+    hipLaunchKernelGGL(kern, dim3(g8 + prm.red_blocks), dim3(64 * NW), Cfg::LDS_BYTES, stream, prm);
   return hipGetLastError() == hipSuccess ? FST_OK : FST_ELAUNCH;
 }
 

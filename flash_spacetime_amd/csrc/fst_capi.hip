@@ -499,41 +499,12 @@ static bwd_dispatch_fn bwd_table(int dtype, int D) {
   return nullptr;
 }
 
-// dW / db from the per-block partials of the rows kernel, in two fixed-order
-// stages so the result does not depend on scheduling: stage 1 sums runs of
-// kRedSeg consecutive blocks per column (coalesced over the columns), stage
-// 2 sums the run totals in four interleaved sums added in order.
-constexpr int kRedSeg = 64;
-
-// Blocks of the call's work list (of `rows` rows).
-__device__ __forceinline__ int total_blocks(const EventSpec& ev, int rows) {
-  if (!ev.inl) return ev.blkcum[ev.B];
-  return __builtin_amdgcn_readlane(InlineList(ev, rows).incl, 63);
-}
-
-// Blocks [64 s, 64 s + 64) of column col, in order.
-__device__ __forceinline__ float run_sum(const float* part, int nblk, int ncol, int s, int col) {
-  const long w0 = (long)s * kRedSeg;
-  const long w1 = w0 + kRedSeg < nblk ? w0 + kRedSeg : nblk;
-  float acc = 0.f;
-#pragma unroll 8
-  for (long w = w0; w < w1; ++w) acc += part[w * ncol + col];
-  return acc;
-}
-
 __global__ __launch_bounds__(256) void dw_reduce_seg_kernel(const float* part, EventSpec ev, int rows, int ncol,
                                                             float* seg) {
   const int nblk = total_blocks(ev, rows);
   const int col = blockIdx.x * 256 + threadIdx.x;
   if (col >= ncol) return;
   seg[(long)blockIdx.y * ncol + col] = run_sum(part, nblk, ncol, blockIdx.y, col);
-}
-
-__device__ __forceinline__ void store_dw(float acc, int e, int DC, float* dw, float* db) {
-  if (e < DC)
-    dw[e] = acc;
-  else if (db)
-    db[e - DC] = acc;
 }
 
 // Stage 2: a workgroup per 64 columns; thread (q, c) sums runs q, q + 4, ...
@@ -552,31 +523,6 @@ __global__ __launch_bounds__(256) void dw_reduce_final_kernel(const float* seg, 
   __syncthreads();
   if (q != 0 || e >= DC + D) return;
   store_dw(((part[0][c] + part[1][c]) + part[2][c]) + part[3][c], e, DC, dw, db);
-}
-
-// Both stages in one launch for at most kRedOne runs (1024 blocks): a
-// workgroup per 64 columns, one thread per (run, column), the run totals
-// exchanged through LDS and added in the two-launch order (bit for bit the
-// same sums). A launch less on calls whose kernels take 15 to 60 us; with
-// more runs the two-launch form spreads them over more workgroups.
-constexpr int kRedOne = 16;
-__global__ __launch_bounds__(64 * kRedOne) void dw_reduce_one_kernel(const float* part, EventSpec ev, int rows,
-                                                                     int nseg, int DC, int D, int use_e, float* dw,
-                                                                     float* db) {
-  __shared__ float run[kRedOne][64];
-  const int c = threadIdx.x & 63, s = threadIdx.x >> 6;
-  const int e = blockIdx.x * 64 + c;
-  const int nblk = total_blocks(ev, rows);  // by whole waves
-  if (s < nseg) run[s][c] = use_e && e < DC + D ? run_sum(part, nblk, DC + D, s, e) : 0.f;
-  __syncthreads();
-  if (s != 0 || e >= DC + D) return;
-  float q4[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    q4[q] = 0.f;
-    for (int k = q; k < nseg; k += 4) q4[q] += run[k][c];
-  }
-  store_dw(((q4[0] + q4[1]) + q4[2]) + q4[3], e, DC, dw, db);
 }
 
 __global__ __launch_bounds__(256) void fill_zero_kernel(float* p, int n) {
@@ -970,25 +916,33 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
     rc = fn(prm, 0, HPR, C, st, (int)lay.grid_r, false, &dummy_rows);
     if (rc != FST_OK) return fail(rc, "backward rows kernel launch failed");
   }
+  // A whole call of few tiles sums dW and db in the cols kernel's launch
+  // (reduce_block); the partials are complete when it starts. At most one
+  // such workgroup per CU: with 264 of them (D = C = 64 past 8 runs) 256
+  // events of 64 tokens, 8 heads, measured 191 -> 193 us.
+  const int red_lg = lay.nseg <= 4 ? 6 : lay.nseg <= 8 ? 5 : 4;
+  const int red_blocks = (((D * C + D + (1 << red_lg) - 1) >> red_lg) + 7) & ~7;  // whole rounds of the eight XCDs
+  const bool fold = phases == FST_BWD_ALL && lay.grid_c > 0 && lay.nseg <= kRedFold && red_blocks <= 256;
+  if (fold) {
+    prm.red_seg = (int)lay.nseg;
+    prm.red_rows = lay.rows_r;
+    prm.red_lg = red_lg;
+    prm.red_blocks = red_blocks;
+  }
   if (phases & FST_PHASE_BWD_COLS) {
     rc = fn(prm, 1, HP, C, st, (int)lay.grid_c, false, &dummy_rows);
     if (rc != FST_OK) return fail(rc, "backward cols kernel launch failed");
   }
-  if (phases & FST_PHASE_REDUCE) {
+  if ((phases & FST_PHASE_REDUCE) && !fold) {
     const int DC = D * C;
     const int ncol = DC + D;
     float* seg = reinterpret_cast<float*>(ws + lay.off_seg);
     if (lay.nseg > 65535) return fail(FST_EUNSUPPORTED, "problem too large for the dW reduction");
-    if (lay.nseg <= kRedOne) {
-      hipLaunchKernelGGL(dw_reduce_one_kernel, dim3((ncol + 63) / 64), dim3(64 * kRedOne), 0, st, prm.dw_part, prm.ev,
-                         lay.rows_r, (int)lay.nseg, DC, D, use_w ? 1 : 0, dweight, dbias);
-    } else {
-      if (use_w)
-        hipLaunchKernelGGL(dw_reduce_seg_kernel, dim3((ncol + 255) / 256, (unsigned)lay.nseg), dim3(256), 0, st,
-                           prm.dw_part, prm.ev, lay.rows_r, ncol, seg);
-      hipLaunchKernelGGL(dw_reduce_final_kernel, dim3((ncol + 63) / 64), dim3(256), 0, st, seg, (int)lay.nseg, DC,
-                         D, use_w ? 1 : 0, dweight, dbias);
-    }
+    if (use_w && lay.nseg > 0)
+      hipLaunchKernelGGL(dw_reduce_seg_kernel, dim3((ncol + 255) / 256, (unsigned)lay.nseg), dim3(256), 0, st,
+                         prm.dw_part, prm.ev, lay.rows_r, ncol, seg);
+    hipLaunchKernelGGL(dw_reduce_final_kernel, dim3((ncol + 63) / 64), dim3(256), 0, st, seg, (int)lay.nseg, DC,
+                       D, use_w ? 1 : 0, dweight, dbias);
     if (hipGetLastError() != hipSuccess) return fail(FST_ELAUNCH, "dW reduction launch failed");
   }
   return FST_OK;

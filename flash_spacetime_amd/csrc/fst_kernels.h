@@ -287,7 +287,74 @@ struct BwdParams {
   float* dweight;
   float* dbias;         // nullable
   FreqTable freq;
+  // dW / db summed by the first red_blocks workgroups of the cols launch
+  // (reduce_block) over red_seg runs of the rows kernel's red_rows-row blocks;
+  // 0: by a launch of their own.
+  int red_blocks, red_seg, red_rows, red_lg;
 };
+
+// dW / db from the per-block partials of the rows kernel, in two fixed-order
+// stages so the result does not depend on scheduling: stage 1 sums runs of
+// kRedSeg consecutive blocks per column (coalesced over the columns), stage
+// 2 sums the run totals in four interleaved sums added in order.
+constexpr int kRedSeg = 64;
+
+// Blocks of the call's work list (of `rows` rows).
+__device__ __forceinline__ int total_blocks(const EventSpec& ev, int rows) {
+  if (!ev.inl) return ev.blkcum[ev.B];
+  return __builtin_amdgcn_readlane(InlineList(ev, rows).incl, 63);
+}
+
+// Blocks [64 s, 64 s + 64) of column col, in order.
+__device__ __forceinline__ float run_sum(const float* part, int nblk, int ncol, int s, int col) {
+  const long w0 = (long)s * kRedSeg;
+  const long w1 = w0 + kRedSeg < nblk ? w0 + kRedSeg : nblk;
+  float acc = 0.f;
+#pragma unroll 8
+  for (long w = w0; w < w1; ++w) acc += part[w * ncol + col];
+  return acc;
+}
+
+__device__ __forceinline__ void store_dw(float acc, int e, int DC, float* dw, float* db) {
+  if (e < DC)
+    dw[e] = acc;
+  else if (db)
+    db[e - DC] = acc;
+}
+
+// Both stages by the first workgroups of the cols kernel's launch, for at most
+// kRedFold runs (1024 blocks): a thread per run and column, 2^red_lg columns a
+// workgroup (64 for up to 4 runs, 32 for up to 8, else 16: every run is summed
+// at once and a workgroup is 256 threads), the run totals exchanged through
+// LDS and added in the two-launch order (bit for bit the same sums). It runs
+// beside the cols tiles, and the launch it saves is 6 us of kernel and the gap
+// before it on calls whose kernels take 15 to 60 us. Whole backward, bf16,
+// D = 32, C = 16, 4 / 12 heads: 16 events of 64 tokens 23.7 -> 18.7 / 29.3 ->
+// 24.5 us, 48 of 192 57.4 -> 52.2 / 90.1 -> 84.6, 256 of 64 48.2 -> 46.1 /
+// 77.4 -> 73.1 (64 columns a workgroup at 16 runs, four runs one after the
+// other: 55.2 / 75.9). With more runs the two launches spread them over more
+// workgroups. part: 1 KB of LDS.
+constexpr int kRedFold = 16;
+template <int DC, int D>
+__device__ void reduce_block(const BwdParams& prm, int tid, float* part) {
+  const int lg = prm.red_lg, nc = 1 << lg, c = tid & (nc - 1), s = tid >> lg;
+  const int e = (blockIdx.x << lg) + c;
+  const bool ok = e < DC + D;
+  const int nblk = total_blocks(prm.ev, prm.red_rows);  // by whole waves
+  if (tid < 256)
+    part[tid] = ok && s < prm.red_seg && (prm.flags & (FST_ATTN_BIAS | FST_ACT_BIAS))
+                    ? run_sum(prm.dw_part, nblk, DC + D, s, e)
+                    : 0.f;
+  __syncthreads();
+  if (s != 0 || !ok) return;
+  float q4[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    q4[q] = 0.f;
+    for (int k = q; k < prm.red_seg; k += 4) q4[q] += part[(k << lg) + c];
+  }
+  store_dw(((q4[0] + q4[1]) + q4[2]) + q4[3], e, DC, prm.dweight, prm.dbias);
+}
 
 template <typename T>
 struct VecOf;

@@ -2,12 +2,13 @@
 
 A whole forward or backward call of at most 64 events has every workgroup
 form the lists it needs (event order, tile counts, sanitised offsets) and,
-for at most 1024 tiles, sums dW / db in one launch; the same phases issued
-one by one build the lists with the work-list kernel and reduce in the same
-order. Both must give the same bits: around the 64-event line (63, 64, 65),
+for at most 1024 tiles, sums dW / db in the cols kernel's launch; the same
+phases issued one by one build the lists with the work-list kernel and reduce
+in the same order in launches of their own. Both must give the same bits: around the 64-event line (63, 64, 65),
 with empty and one-token events, padded and packed, both dtypes, and with
-malformed packed offsets (NaN from both). Past the one-launch reduction
-(more than 1024 tiles) dW and db are checked the same way.
+malformed packed offsets (NaN from both). Each width of
+the reduction's workgroups (up to 4, 8 and 16 runs of 64 tiles), and the calls
+past it (more runs, or more workgroups than CUs), are checked the same way.
 """
 
 import pytest
@@ -31,6 +32,13 @@ CASES = [
     (torch.bfloat16, 8, 32, 16, [0, 16, 1, 17, 33, 0, 48, 2, 15], False),
     (torch.bfloat16, 8, 48, 48, [1, 0, 40], True),
     (torch.bfloat16, 2, 16, 16, [300] * 60, False),       # more than 1024 tiles
+    (torch.bfloat16, 4, 16, 32, [200] * 20 + [1], False),  # 261 tiles: 5 runs
+    (torch.bfloat16, 2, 48, 16, [250] * 32, True),         # 512 tiles: 8 runs
+    (torch.bfloat16, 2, 16, 48, [190, 0, 200] * 15, False),  # 375 tiles: 6 runs
+    (torch.bfloat16, 2, 64, 48, [256] * 64, False),        # 1024 tiles: 16 runs, 200 workgroups
+    (torch.bfloat16, 2, 64, 64, [256] * 33, True),         # 9 runs, too many workgroups
+    (torch.float32, 2, 16, 32, [250] * 40, False),
+    (torch.float32, 8, 64, 64, [33] * 5, True),
     (torch.float32, 4, 16, 16, [0, 31, 1, 17], False),
     (torch.float32, 8, 32, 16, LENS64, True),
     (torch.float32, 12, 32, 16, [64, 0, 5], False),
