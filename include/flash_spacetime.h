@@ -130,7 +130,9 @@ enum fst_flags {
 /* Phases of one operator call, for callers that time or schedule them
  * separately (the one-shot entry points run all of them, in this order).
  * The work list (per-event row-block prefix sums) is written into the
- * workspace by the first phase and read by the later ones. */
+ * workspace by the first phase and read by the later ones; a call of all
+ * phases at once may form it, and sum the partials, inside the other phases'
+ * kernels instead (calls of few events or tiles; the same results). */
 enum fst_phase {
   FST_PHASE_WORKLIST = 1, /* per-event row blocks -> workspace (tiny kernel)   */
   FST_PHASE_FWD = 2,      /* forward kernel                                   */
