@@ -679,10 +679,11 @@ int fst_forward_phases(int phases, int dtype, int flags, int B, int H, int L, in
 
   const WorkList wl = worklist_at(workspace, B);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // A whole call of few events needs no work list (InlineList); phases run
-  // one by one keep it.
-  const bool inl = B <= kInlineEvents && phases == FST_FWD_ALL;
-  if ((phases & FST_PHASE_WORKLIST) && !inl) {
+  // With few events the forward kernel forms the list it needs (InlineList),
+  // whichever phases ran on the workspace before; a whole call then launches
+  // no work-list kernel.
+  const bool inl = B <= kInlineEvents;
+  if ((phases & FST_PHASE_WORKLIST) && !(inl && phases == FST_FWD_ALL)) {
     if (launch_worklist(lens, packed, B, L, T, rows, wl.blkcum, 0, nullptr, wl.perm, wl.scum, nullptr, wl.cus,
                         wl.status, st) != FST_OK)
       return fail(FST_ELAUNCH, "work-list kernel launch failed");
@@ -854,8 +855,8 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
   // The bf16 rows kernel's padding-last schedule (16-row tiles, padded events).
   int32_t* vp = (dtype == FST_BF16 && !packed && lay.rows_r == 16) ? reinterpret_cast<int32_t*>(ws + lay.off_vp)
                                                                     : nullptr;
-  const bool inl = B <= kInlineEvents && phases == FST_BWD_ALL;  // as in the forward
-  if ((phases & FST_PHASE_WORKLIST) && !inl) {
+  const bool inl = B <= kInlineEvents;  // as in the forward
+  if ((phases & FST_PHASE_WORKLIST) && !(inl && phases == FST_BWD_ALL)) {
     if (launch_worklist(lens, packed, B, L, T, lay.rows_r, wr.blkcum, lay.rows_c, wc.blkcum, wr.perm, wr.scum,
                         wc.scum, wr.cus, wr.status, st, vp) != FST_OK)
       return fail(FST_ELAUNCH, "work-list kernel launch failed");

@@ -3,10 +3,12 @@
 A whole forward or backward call of at most 64 events has every workgroup
 form the lists it needs (event order, tile counts, sanitised offsets) and,
 for at most 1024 tiles, sums dW / db in the cols kernel's launch; the same
-phases issued one by one build the lists with the work-list kernel and reduce
-in the same order in launches of their own. Both must give the same bits: around the 64-event line (63, 64, 65),
-with empty and one-token events, padded and packed, both dtypes, and with
-malformed packed offsets (NaN from both). Each width of
+phases issued one by one form the same lists (read them past 64 events) and
+reduce in the same order in launches of their own. Both must give the same
+bits: around the 64-event line (63, 64, 65), with empty and one-token events,
+padded and packed, both dtypes, and with malformed packed offsets (NaN from
+both). test_phase_order_gpu.py compares the lists the workgroups form with
+those the work-list kernel writes. Each width of
 the reduction's workgroups (up to 4, 8 and 16 runs of 64 tiles), and the calls
 past it (more runs, or more workgroups than CUs), are checked the same way.
 """
