@@ -138,7 +138,7 @@ def host():
             raise LibraryMissing(f"{e}: build it with `python -m flash_spacetime_amd.build`") from e
         _fst_host.bind_library(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in (
             "fst_supported", "fst_forward_workspace_bytes", "fst_forward", "fst_backward_workspace_bytes",
-            "fst_backward")))
+            "fst_backward", "fst_last_error")))
         _HOST = _fst_host
     return _HOST
 

@@ -677,6 +677,12 @@ int fst_forward_phases(int phases, int dtype, int flags, int B, int H, int L, in
     return fail(FST_EUNSUPPORTED, "no compiled forward kernel for dtype=%d H=%d D=%d C=%d with plan bits 0x%x", dtype,
                 H, D, C, flags & FST_PLAN_MASK);
 
+  // Padded grids cover ceil(B / 8) * 8 events (the tile kernels' schedule
+  // deals events to the eight XCDs); workgroups without work exit at once.
+  // Refusals come before the first launch.
+  const long grid = packed ? ((long)T + rows - 1) / rows + B : (long)((B + 7) / 8 * 8) * ((L + rows - 1) / rows);
+  if ((phases & FST_PHASE_FWD) && grid > 0x7fffffffL) return fail(FST_EUNSUPPORTED, "problem too large for one launch");
+
   const WorkList wl = worklist_at(workspace, B);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // With few events the forward kernel forms the list it needs (InlineList),
@@ -719,10 +725,6 @@ int fst_forward_phases(int phases, int dtype, int flags, int B, int H, int L, in
   prm.out = out;
   prm.lse = lse;
   freq_table(C, prm.freq);
-  // Padded grids cover ceil(B / 8) * 8 events (the tile kernels' schedule
-  // deals events to the eight XCDs); workgroups without work exit at once.
-  const long grid = packed ? ((long)T + rows - 1) / rows + B : (long)((B + 7) / 8 * 8) * ((L + rows - 1) / rows);
-  if (grid > 0x7fffffffL) return fail(FST_EUNSUPPORTED, "problem too large for one launch");
   rc = fn(prm, HP, C, st, (int)grid, false, &rows);
   if (rc != FST_OK) return fail(rc, "forward kernel launch failed (%s)", hipGetErrorString(hipGetLastError()));
   return FST_OK;
@@ -848,7 +850,10 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
     return fail(FST_EUNSUPPORTED, "no compiled backward for dtype=%d H=%d D=%d C=%d", dtype, H, D, C);
   if (!workspace || workspace_bytes < lay.total)
     return fail(FST_EWORKSPACE, "workspace of %zu bytes is smaller than the %zu required", workspace_bytes, lay.total);
+  // Refusals come before the first launch.
   if (lay.grid_r > 0x7fffffffL || lay.grid_c > 0x7fffffffL) return fail(FST_EUNSUPPORTED, "problem too large");
+  if ((phases & FST_PHASE_REDUCE) && lay.nseg > 65535)
+    return fail(FST_EUNSUPPORTED, "problem too large for the dW reduction");
 
   unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
   const WorkList wr = worklist_at(ws + lay.off_bc_r, B), wc = worklist_at(ws + lay.off_bc_c, B);
@@ -938,7 +943,6 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
     const int DC = D * C;
     const int ncol = DC + D;
     float* seg = reinterpret_cast<float*>(ws + lay.off_seg);
-    if (lay.nseg > 65535) return fail(FST_EUNSUPPORTED, "problem too large for the dW reduction");
     if (use_w && lay.nseg > 0)
       hipLaunchKernelGGL(dw_reduce_seg_kernel, dim3((ncol + 255) / 256, (unsigned)lay.nseg), dim3(256), 0, st,
                          prm.dw_part, prm.ev, lay.rows_r, ncol, seg);

@@ -9,15 +9,19 @@
 // Both functions return None for anything but that form (unsupported shapes
 // and dtypes, mixed devices, tensor subclasses, lengths that are not integers
 // on the device, heads in groups, a call the library refuses): the caller then
-// takes the Python path, which handles or rejects it. Nothing is launched
-// before the decision. Nothing is kept between calls but the library's entry
-// points.
+// takes the Python path, which handles or rejects it. The library refuses
+// before it launches a kernel; operands may have been converted by then. A
+// call that failed otherwise (a launch error, a pending error of the device)
+// raises: it is not run a second time. Nothing is kept between calls but the
+// library's entry points.
 #include <torch/extension.h>
 
 #include <ATen/TensorSubclassLikeUtils.h>
 
 #include <cmath>
 #include <optional>
+#include <stdexcept>
+#include <string>
 
 #include "../../include/flash_spacetime.h"
 
@@ -32,14 +36,24 @@ struct Library {
   decltype(&fst_forward) forward = nullptr;
   decltype(&fst_backward_workspace_bytes) backward_workspace_bytes = nullptr;
   decltype(&fst_backward) backward = nullptr;
+  decltype(&fst_last_error) last_error = nullptr;
 } lib;
 
-void bind_library(size_t supported, size_t fwd_ws, size_t fwd, size_t bwd_ws, size_t bwd) {
+void bind_library(size_t supported, size_t fwd_ws, size_t fwd, size_t bwd_ws, size_t bwd, size_t last_error) {
   lib.supported = reinterpret_cast<decltype(lib.supported)>(supported);
   lib.forward_workspace_bytes = reinterpret_cast<decltype(lib.forward_workspace_bytes)>(fwd_ws);
   lib.forward = reinterpret_cast<decltype(lib.forward)>(fwd);
   lib.backward_workspace_bytes = reinterpret_cast<decltype(lib.backward_workspace_bytes)>(bwd_ws);
   lib.backward = reinterpret_cast<decltype(lib.backward)>(bwd);
+  lib.last_error = reinterpret_cast<decltype(lib.last_error)>(last_error);
+}
+
+// Whether the library refused the call (a status it returns before any
+// launch); any other failure raises with the library's message.
+bool refused(int rc, const char* what) {
+  if (rc == FST_EINVAL || rc == FST_EUNSUPPORTED) return true;
+  if (rc != FST_OK) throw std::runtime_error(std::string(what) + ": " + lib.last_error());
+  return false;
 }
 
 // A plain strided tensor on `dev`: no subclass, functorch wrapper, lazy
@@ -139,7 +153,7 @@ py::object forward_call(const Tensor& q_in, const std::optional<Tensor>& k_in, c
                      static_cast<const float*>(data(b32)), static_cast<const int32_t*>(data(len32)), (float)sc,
                      data(out), static_cast<float*>(data(lse)), data(ws), bytes, reinterpret_cast<void*>(stream));
   }
-  if (rc != FST_OK) return py::none();
+  if (refused(rc, "flash_spacetime_forward")) return py::none();
   return py::make_tuple(out, lse, qc, kc, vc, pos4, w32, bias.has_value() ? py::cast(b32) : py::none(), len32,
                         py::make_tuple(dtype, flags, B, H, L, T, D, C), sc);
 }
@@ -226,17 +240,17 @@ py::object backward_call(const Dims& dims, const Tensor& q_in, const std::option
       static_cast<float*>(data(dw)), static_cast<float*>(data(db)), nullptr, data(ws), bytes,
       reinterpret_cast<void*>(stream));
   }
-  if (rc != FST_OK) return py::none();
+  if (refused(rc, "flash_spacetime_backward")) return py::none();
   return py::make_tuple(inter ? grad : dq, inter ? Tensor() : dk, inter ? Tensor() : dv, dw, b32.has_value() ? py::cast(db) : py::none());
 }
 
-// A failed allocation (or any other tensor error) is the Python path's to
-// report: it frees nothing here and raises there as it always did.
+// A failed allocation is the Python path's to report, with the exception type
+// torch gives it there. Any other tensor error raises here.
 template <typename F, typename... A>
 py::object or_none(F f, const A&... args) {
   try {
     return f(args...);
-  } catch (const c10::Error&) {
+  } catch (const c10::OutOfMemoryError&) {
     return py::none();
   }
 }

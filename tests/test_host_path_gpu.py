@@ -8,8 +8,12 @@ lengths, features, weight and bias, absent bias, head groups, both dtypes.
 What the Python path refuses stays refused with its exception.
 """
 
+import ctypes
+
 import pytest
 import torch
+
+from flash_spacetime_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -174,3 +178,44 @@ def test_refused_calls_stay_refused():
     with pytest.raises((AttributeError, TypeError, ValueError)):
         flash_spacetime_attention_varlen(_draw(sum(LENS), 3, 4, D), None, None, _draw(sum(LENS), 5, dtype=torch.float32),
                                          w, b, torch.tensor([0, 54], device=DEV, dtype=torch.int32))
+
+
+# The library's entry points replaced by host functions that return a status
+# (nothing is launched): what the operators make of it.
+_ENTRY = ("fst_supported", "fst_forward_workspace_bytes", "fst_forward", "fst_backward_workspace_bytes",
+          "fst_backward", "fst_last_error")
+
+
+def _bind(**stubs):
+    lib = _lib.load()
+    _lib.host().bind_library(*(ctypes.cast(stubs.get(n, getattr(lib, n)), ctypes.c_void_p).value for n in _ENTRY))
+
+
+def _returning(name, status, calls):
+    res, args = _lib.SIGNATURES[name]
+
+    def entry(*_):
+        calls.append(name)
+        return status
+
+    return ctypes.CFUNCTYPE(res, *args)(entry)
+
+
+@pytest.mark.parametrize("name", ["fst_forward", "fst_backward"])
+@pytest.mark.parametrize("status", [_lib.FST_ELAUNCH, _lib.FST_EWORKSPACE, _lib.FST_EUNSUPPORTED, _lib.FST_EINVAL])
+def test_failed_calls_raise_and_refused_ones_take_the_python_path(name, status):
+    """A launch error is reported, not hidden by a second run of the call; a
+    call the library refuses is left to the Python path (which here runs it)."""
+    calls, want = [], _run("packed")
+    stub = _returning(name, status, calls)
+    try:
+        _bind(**{name: stub})
+        if status in (_lib.FST_ELAUNCH, _lib.FST_EWORKSPACE):
+            with pytest.raises(RuntimeError, match="flash_spacetime_" + name[4:]):
+                _run("packed")
+        else:
+            assert all(torch.equal(a, e) for a, e in zip(_run("packed"), want))
+    finally:
+        _bind()
+    assert calls == [name]
+    assert all(torch.equal(a, e) for a, e in zip(_run("packed"), want))
