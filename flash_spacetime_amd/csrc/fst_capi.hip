@@ -361,6 +361,22 @@ static int launch_worklist(const int32_t* lens, bool packed, int B, int L, int T
   return hipGetLastError() == hipSuccess ? FST_OK : FST_ELAUNCH;
 }
 
+// Whether a call's kernels form the work list themselves (InlineList): a rule
+// on the call's sizes alone, so that phases run one by one agree with a whole
+// call. A call of up to 64 events saves the work-list kernel and its launch,
+// 2.5 to 6 us a direction, and pays in every workgroup for finding its tile, in
+// the bf16 kernels by ranking the events; the cost grows with events times
+// tiles. B events padded to L, all of 16 tokens (the worst case: nothing else to
+// do), D = 32, C = 16, H = 12, bf16, backward with the list / without: B = 16,
+// L = 1500 31.7 / 28.2 us, B = 64, L = 192 25.6 / 21.4 (49152 events times
+// tiles), B = 32, L = 1500 40.1 / 41.7 (96256), B = 64, L = 768 43.6 / 51.1,
+// L = 3000 116 / 150; float32 (no ranking), H = 2, D = C = 16: B = 64, L = 768
+// 57.8 / 53.4, L = 1500 87.4 / 83.9 (385024).
+static bool inline_list(int dtype, bool packed, int B, int L, int T) {
+  const long tiles = packed ? (long)T / 16 + B : (long)((B + 7) / 8 * 8) * ((L + 15) / 16);
+  return B <= kInlineEvents && B * tiles <= (dtype == FST_BF16 ? 1L << 16 : 1L << 18);
+}
+
 typedef int (*fwd_dispatch_fn)(const FwdParams&, int, int, hipStream_t, int, bool, int*);
 
 static fwd_dispatch_fn fwd_table(int dtype, int D) {
@@ -685,10 +701,10 @@ int fst_forward_phases(int phases, int dtype, int flags, int B, int H, int L, in
 
   const WorkList wl = worklist_at(workspace, B);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // With few events the forward kernel forms the list it needs (InlineList),
-  // whichever phases ran on the workspace before; a whole call then launches
-  // no work-list kernel.
-  const bool inl = B <= kInlineEvents;
+  // Where the forward kernel forms the list it needs, it does so whichever
+  // phases ran on the workspace before; a whole call then launches no
+  // work-list kernel.
+  const bool inl = inline_list(dtype, packed, B, L, T);
   if ((phases & FST_PHASE_WORKLIST) && !(inl && phases == FST_FWD_ALL)) {
     if (launch_worklist(lens, packed, B, L, T, rows, wl.blkcum, 0, nullptr, wl.perm, wl.scum, nullptr, wl.cus,
                         wl.status, st) != FST_OK)
@@ -860,7 +876,7 @@ int fst_backward_phases(int phases, int dtype, int flags, int B, int H, int L, i
   // The bf16 rows kernel's padding-last schedule (16-row tiles, padded events).
   int32_t* vp = (dtype == FST_BF16 && !packed && lay.rows_r == 16) ? reinterpret_cast<int32_t*>(ws + lay.off_vp)
                                                                     : nullptr;
-  const bool inl = B <= kInlineEvents;  // as in the forward
+  const bool inl = inline_list(dtype, packed, B, L, T);  // as in the forward
   if ((phases & FST_PHASE_WORKLIST) && !(inl && phases == FST_BWD_ALL)) {
     if (launch_worklist(lens, packed, B, L, T, lay.rows_r, wr.blkcum, lay.rows_c, wc.blkcum, wr.perm, wr.scum,
                         wc.scum, wr.cus, wr.status, st, vp) != FST_OK)

@@ -28,7 +28,8 @@ struct EventSpec {
   int max_len;            // longest event whose rows of all heads span less than 2^31 bytes
   // No work list: lens are the caller's (the raw cu_seqlens when packed) and
   // every workgroup forms the lists it needs itself (InlineList); blkcum,
-  // perm, scum, vp and status are null. Calls of up to kInlineEvents events.
+  // perm, scum, vp and status are null. Calls of up to kInlineEvents events
+  // (fst_capi.hip: inline_list).
   int inl;
 };
 
@@ -131,10 +132,12 @@ __device__ __forceinline__ int wave_scan(int x, int id, Op op) {
 
 // The work list of a call of at most kInlineEvents events, formed by each
 // wave for itself: lane i holds event i. Sanitised token ranges, block counts
-// and the offsets' verdict are those worklist_kernel writes. A call that small
-// spent 7 us in the work-list kernel plus the launch before each direction's
-// first kernel; the wave's own list takes two loads, some forty vector
-// instructions and, for the schedules, five per event.
+// and the offsets' verdict are those worklist_kernel writes. The wave's own
+// list takes two loads, some forty vector instructions and, for the schedules,
+// a rank per event (three instructions an event; ranking and summing the
+// blocks before each event took ten, and three waves a SIMD run it: forward of
+// 64 events of up to 192 tokens, H = 12, D = C = 32, bf16 33.8 us, with the list
+// 31.6).
 constexpr int kInlineEvents = 64;
 struct InlineList {
   int tok0, len, nblk, incl;  // this lane's event; incl: blocks of events 0 .. lane
@@ -159,18 +162,21 @@ struct InlineList {
     nblk = !in ? 0 : (len > 0 ? (len + rows - 1) / rows : (ev.packed ? 0 : 1));
     incl = wave_scan(nblk, 0, [](int a, int c) { return a + c; });
   }
-  // Position of this lane's event by decreasing length (ties by index), and
-  // the blocks of the events before it in that order.
-  __device__ __forceinline__ void order(int B, int& rank, int& before) const {
+  // Position of this lane's event by decreasing length (ties by index): the
+  // count of larger keys among the first B, eight to a step (lanes past the
+  // events hold the lowest key; their own rank is B).
+  __device__ __forceinline__ int rank(int B) const {
     const int lane = threadIdx.x & 63;
-    rank = before = 0;
-    for (int j = 0; j < B; ++j) {
-      const int lj = __builtin_amdgcn_readlane(len, j), nj = __builtin_amdgcn_readlane(nblk, j);
-      const bool first = lj > len || (lj == len && j < lane);
-      rank += first ? 1 : 0;
-      before += first ? nj : 0;
-    }
+    const int key = lane < B ? (min(len, (1 << 25) - 1) << 6) | (63 - lane) : -1;
+    int r = 0;
+    for (int j = 0; j < B; j += 8)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) r += __builtin_amdgcn_readlane(key, j + i) > key ? 1 : 0;
+    return r;
   }
+  // Blocks of the event in position `lane` of the order that rank() gives (0
+  // past the events).
+  __device__ __forceinline__ int by_rank(int r) const { return __builtin_amdgcn_ds_permute(r << 2, nblk); }
   // Lane b's event as eb.
   __device__ __forceinline__ void event(int b, EventBlock& eb) const {
     eb.b = b;
@@ -180,6 +186,9 @@ struct InlineList {
     eb.bad = bad;
   }
 };
+__device__ __forceinline__ int wave_sum_scan(int x) {
+  return wave_scan(x, 0, [](int a, int c) { return a + c; });
+}
 // The lane a ballot names (one bit set).
 __device__ __forceinline__ int ballot_lane(bool hit) { return __builtin_ctzll(__builtin_amdgcn_ballot_w64(hit)); }
 

@@ -179,44 +179,54 @@ struct DTiles {
 // wave's own list; padlast stands for ev.vp there.
 __device__ __forceinline__ bool inline_tile_block(const EventSpec& ev, bool padlast, int w, EventBlock& eb) {
   const InlineList il(ev, 16);
-  int rank, before;
-  il.order(ev.B, rank, before);
+  const int rank = il.rank(ev.B);
   const int lane = threadIdx.x & 63;
   const bool in = lane < ev.B;
   const int x = w & 7, k = w >> 3;
+  // The event in position p of the order.
+  auto take = [&](int p) __attribute__((always_inline)) { il.event(ballot_lane(in && rank == p), eb); };
+  // Where entry t of the concatenated counts c (one per position) falls: its
+  // position, with t reduced to the index within it; -1 past them all.
+  auto find = [&](int c, int& t) __attribute__((always_inline)) {
+    const int first = wave_sum_scan(c) - c;
+    const unsigned long long hit = __builtin_amdgcn_ballot_w64(t >= first && t < first + c);
+    if (hit == 0) return -1;
+    const int p = __builtin_ctzll(hit);
+    t -= __builtin_amdgcn_readlane(first, p);
+    return p;
+  };
   if (ev.packed) {
-    const int t = (((k >> 3) << 3) + x) * 8 + (k & 7);
-    const bool hit = in && t >= before && t < before + il.nblk;
-    if (__builtin_amdgcn_ballot_w64(hit) == 0) return false;
-    const int b = ballot_lane(hit);
-    il.event(b, eb);
-    eb.blk = t - __builtin_amdgcn_readlane(before, b);
+    int t = (((k >> 3) << 3) + x) * 8 + (k & 7);
+    const int p = find(il.by_rank(rank), t);
+    if (p < 0) return false;
+    take(p);
+    eb.blk = t;
     return true;
   }
   const int nb = (ev.L + 15) >> 4;
-  // The XCD's events in order: rank 8 j + (j odd ? 7 - x : x).
-  auto nth = [&](int j) __attribute__((always_inline)) { return 8 * j + ((j & 1) ? 7 - x : x); };
   if (!padlast) {
-    const int j = k / nb, r = nth(j);
+    // The XCD's j-th event: position 8 j + (j odd ? 7 - x : x).
+    const int j = k / nb, r = 8 * j + ((j & 1) ? 7 - x : x);
     if (r >= ev.B) return false;
-    il.event(ballot_lane(in && rank == r), eb);
+    take(r);
     eb.blk = k - j * nb;
     return true;
   }
-  // Valid tiles first, then the padding-only ones.
-  int rem = k;
-  for (int pass = 0; pass < 2; ++pass)
-    for (int j = 0; nth(j) < ev.B; ++j) {
-      const int b = ballot_lane(in && rank == nth(j));
-      const int v = __builtin_amdgcn_readlane(il.nblk, b), c = pass == 0 ? v : nb - v;
-      if (rem < c) {
-        il.event(b, eb);
-        eb.blk = pass == 0 ? rem : v + rem;
-        return true;
-      }
-      rem -= c;
-    }
-  return false;
+  // The XCD's valid tiles first, then its padding-only ones.
+  const bool mine = in && (((lane >> 3) & 1) ? 7 - (lane & 7) : lane & 7) == x;
+  const int v = il.by_rank(rank);
+  int t = k, p = find(mine ? v : 0, t);
+  if (p >= 0) {
+    take(p);
+    eb.blk = t;
+    return true;
+  }
+  t -= __builtin_amdgcn_readlane(wave_sum_scan(mine ? v : 0), 63);
+  p = find(mine ? nb - v : 0, t);
+  if (p < 0) return false;
+  take(p);
+  eb.blk = __builtin_amdgcn_readlane(v, p) + t;
+  return true;
 }
 
 __device__ __forceinline__ bool tile_block(const EventSpec& ev, bool padlast, int w, EventBlock& eb) {

@@ -130,11 +130,11 @@ enum fst_flags {
 /* Phases of one operator call, for callers that time or schedule them
  * separately (the one-shot entry points run all of them, in this order).
  * The work list (per-event row-block prefix sums) is written into the
- * workspace by the first phase and read by the later ones. In calls of at
- * most 64 events the later phases form it from lens themselves (the same
- * list), and a call of all phases at once leaves it unwritten. Once the
- * first phase, or a call of all phases at once, has run on a workspace, the
- * later phases may run on it again one by one with the same arguments. A
+ * workspace by the first phase and read by the later ones. In calls of few
+ * events (at most 64) and tiles the later phases form it from lens themselves
+ * (the same list), and a call of all phases at once leaves it unwritten. Once
+ * the first phase, or a call of all phases at once, has run on a workspace,
+ * the later phases may run on it again one by one with the same arguments. A
  * call of all phases at once of few tiles sums the partials inside the cols
  * kernel's launch (the same sums). */
 enum fst_phase {

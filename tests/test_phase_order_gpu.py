@@ -7,8 +7,8 @@ padded and packed, with the dW / db sums in the cols kernel's launch and in
 launches of their own. The workspaces start as zeros, which a kernel that
 read an unwritten list would take for a list of no work.
 
-Up to 64 events the kernels form the work list themselves; with empty events
-appended past 64 the work-list kernel writes it. The events' rows must be the
+Up to 64 events of few tiles the kernels form the work list themselves; with
+empty events appended past 64 the work-list kernel writes it. The events' rows must be the
 same bits either way, and so must dW and db (an empty event adds zeros after
 the others' partial sums). Malformed packed offsets must be refused alike.
 """
@@ -30,7 +30,9 @@ CASES = [
     (torch.bfloat16, 12, 32, 16, [33, 0, 17], True),
     (torch.bfloat16, 3, 16, 16, LENS64, False),
     (torch.bfloat16, 2, 16, 16, LENS64 + [5], True),       # 65 events: a written list
-    (torch.bfloat16, 2, 16, 16, [300] * 60, False),        # dW / db in launches of their own
+    (torch.bfloat16, 2, 16, 16, [300] * 60, False),        # too many tiles: a written list, dW / db in launches of their own
+    (torch.bfloat16, 4, 16, 16, [700, 40, 0, 655, 16] * 3, False),  # padding-only tiles of many lengths
+    (torch.bfloat16, 2, 16, 16, [1000] + LENS64[1:], True),
     (torch.float32, 12, 32, 16, [40, 0, 7], False),
     (torch.float32, 4, 16, 32, LENS64, True),
 ]

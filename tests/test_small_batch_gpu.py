@@ -1,9 +1,9 @@
 """GPU tests of calls of few events, which run without a work-list kernel.
 
-A whole forward or backward call of at most 64 events has every workgroup
-form the lists it needs (event order, tile counts, sanitised offsets) and,
-for at most 1024 tiles, sums dW / db in the cols kernel's launch; the same
-phases issued one by one form the same lists (read them past 64 events) and
+A whole forward or backward call of at most 64 events (and few tiles) has every
+workgroup form the lists it needs (event order, tile counts, sanitised
+offsets) and, for at most 1024 tiles, sums dW / db in the cols kernel's launch; the same
+phases issued one by one form the same lists (else read them) and
 reduce in the same order in launches of their own. Both must give the same
 bits: around the 64-event line (63, 64, 65), with empty and one-token events,
 padded and packed, both dtypes, and with malformed packed offsets (NaN from
