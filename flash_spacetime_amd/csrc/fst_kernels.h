@@ -15,7 +15,7 @@ struct EventSpec {
   const int32_t* lens;    // seqlens [B] (padded) or the work list's sanitised cu_seqlens [B+1] (packed)
   const int32_t* blkcum;  // [B+1] prefix sums of row blocks per event
   const int32_t* perm;    // [B] events by decreasing length (the tile kernels' schedules)
-  const int32_t* scum;    // [B+1] packed: prefix sums of row blocks in perm order (or null)
+  const int32_t* scum;    // [B+1] packed: prefix sums of row blocks in perm order; padded: null
   // [8 ceil(B / 8) + 1] padded: prefix sums of the valid (not padding-only)
   // 16-row tiles over the events in XCD order (entry x S + j: XCD x's j-th
   // event, S = ceil(B / 8)), for tile_block's padding-last schedule; or null.
@@ -268,7 +268,7 @@ struct FwdParams {
 struct BwdParams {
   EventSpec ev;     // rows-kernel work list in ev.blkcum
   const int32_t* blkcum_cols;  // cols-kernel work list
-  const int32_t* scum_cols;    // its packed schedule (row blocks in ev.perm order), or null
+  const int32_t* scum_cols;    // its packed schedule (row blocks in ev.perm order); padded: null
   int H, flags;
   float scale;
   const void *q, *k, *v, *dout;

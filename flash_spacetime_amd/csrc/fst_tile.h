@@ -30,12 +30,6 @@ namespace fst {
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-// Hardware workgroup w of a grid of G (a multiple of 8) runs logical block
-// (w % 8) * (G / 8) + w / 8: workgroups are dealt to the eight XCDs round
-// robin, so each XCD gets a contiguous range of logical blocks and an event's
-// row blocks share one L2.
-__device__ __forceinline__ int xcd_remap(int w, int G) { return (w & 7) * (G >> 3) + (w >> 3); }
-
 // Natural channel index of channel slot k (see the header comment).
 template <int C>
 __host__ __device__ constexpr int slot_channel(int k) {
@@ -233,7 +227,6 @@ __device__ __forceinline__ bool tile_block(const EventSpec& ev, bool padlast, in
   if (ev.inl) return inline_tile_block(ev, padlast, w, eb);
   eb.bad = false;
   if (ev.packed) {
-    if (!ev.scum) return locate_block(ev, 16, xcd_remap(w, gridDim.x), eb);
     const int x = w & 7, k = w >> 3;
     const int t = (((k >> 3) << 3) + x) * 8 + (k & 7);
     if (t >= ev.scum[ev.B]) return false;
