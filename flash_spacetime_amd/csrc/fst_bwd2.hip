@@ -914,7 +914,12 @@ struct Cols2Cfg {
 };
 
 
-template <int HP, int D, int C, int RC, int FL, int OCC, int NW>
+// RED: the launch's first workgroups sum dW / db (reduce_block); the tiles'
+// kernel without that code is an instance of its own, because beside it the
+// compiler gave some tiles two registers more, at the edge of a wave per SIMD
+// (H = 12, D = 16, activation bias only, B = 128, L = 768, lengths U{16..768}:
+// C = 16 0.188 -> 0.202 ms, C = 64 0.340 -> 0.387).
+template <int HP, int D, int C, int RC, int FL, int OCC, int NW, bool RED>
 __global__ __launch_bounds__(64 * NW, OCC) void bwd_cols2_kernel(BwdParams prm) {
   using Cfg = Cols2Cfg<HP, D, C, RC, NW, OCC>;
   using DT = DTiles<D>;
@@ -938,16 +943,20 @@ __global__ __launch_bounds__(64 * NW, OCC) void bwd_cols2_kernel(BwdParams prm) 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
 
-  if ((int)blockIdx.x < prm.red_blocks) {
-    reduce_block<D * C, D>(prm, tid, reinterpret_cast<float*>(smem));
-    return;
+  int wg = blockIdx.x;
+  if constexpr (RED) {
+    if (wg < prm.red_blocks) {
+      reduce_block<D * C, D>(prm, tid, reinterpret_cast<float*>(smem));
+      return;
+    }
+    wg -= prm.red_blocks;
   }
   EventSpec ev = prm.ev;
   ev.blkcum = prm.blkcum_cols;
   ev.scum = prm.scum_cols;
   EventBlock eb;
   // The interleaved schedule (the padding-last one is the rows kernel's).
-  if (!tile_block(ev, false, blockIdx.x - prm.red_blocks, eb)) return;
+  if (!tile_block(ev, false, wg, eb)) return;
   const int len = eb.len;
   const int H = prm.H;
   // FL >= 0: the bias flags fixed at compile time; -1: read at run time.
@@ -1437,10 +1446,14 @@ int bwd2_launch_cols(const BwdParams& prm, hipStream_t stream, int g8, bool quer
   // One instance per bias-flag combination: a kernel reading the flags at
   // run time keeps both bias paths live and spills at the larger layouts.
   const int fl = prm.flags & 3;
-  auto kern = fl == 3   ? bwd_cols2_kernel<HP, D, C, P::RC, 3, OCC, NW>
-              : fl == 1 ? bwd_cols2_kernel<HP, D, C, P::RC, 1, OCC, NW>
-              : fl == 2 ? bwd_cols2_kernel<HP, D, C, P::RC, 2, OCC, NW>
-                        : bwd_cols2_kernel<HP, D, C, P::RC, 0, OCC, NW>;
+  auto pick = [&](auto red) {
+    constexpr bool RED = decltype(red)::value;
+    return fl == 3   ? bwd_cols2_kernel<HP, D, C, P::RC, 3, OCC, NW, RED>
+           : fl == 1 ? bwd_cols2_kernel<HP, D, C, P::RC, 1, OCC, NW, RED>
+           : fl == 2 ? bwd_cols2_kernel<HP, D, C, P::RC, 2, OCC, NW, RED>
+                     : bwd_cols2_kernel<HP, D, C, P::RC, 0, OCC, NW, RED>;
+  };
+  auto kern = prm.red_blocks > 0 ? pick(std::true_type{}) : pick(std::false_type{});
   if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES) !=
       hipSuccess)
     return FST_ELAUNCH;
