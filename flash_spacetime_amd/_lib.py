@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from pathlib import Path
 
 import torch
@@ -127,20 +128,37 @@ def load() -> ctypes.CDLL:
 _HOST = None
 
 
+def _load_host():
+    """The host extension bound to the loaded library, or False (with a warning
+    that says why) where it is not built, or was built for another torch or
+    with another library than the one loaded: the operators then launch the
+    same kernels through ctypes, some 20 to 50 us a direction slower."""
+    lib = load()
+    build = lib.fst_version().decode().split(" build ")[-1]
+    try:
+        from . import _fst_host
+    except ImportError as e:
+        why = str(e)
+    else:
+        have = (_fst_host.build_id, _fst_host.torch_version)
+        if have == (build, torch.__version__):
+            _fst_host.bind_library(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in (
+                "fst_supported", "fst_forward_workspace_bytes", "fst_forward", "fst_backward_workspace_bytes",
+                "fst_backward", "fst_last_error")))
+            return _fst_host
+        why = f"it is build {have[0]} for torch {have[1]}, the library is build {build} and torch is {torch.__version__}"
+    warnings.warn(f"the host extension _fst_host is not used ({why}); the operators run through ctypes. "
+                  "Rebuild with `python -m flash_spacetime_amd.build`", RuntimeWarning, stacklevel=4)
+    return False
+
+
 def host():
-    """The host extension (csrc/fst_host.cpp), bound once to the loaded library."""
+    """The host extension (csrc/fst_host.cpp), looked up and bound once; None
+    where it cannot be used (_load_host)."""
     global _HOST
     if _HOST is None:
-        lib = load()
-        try:
-            from . import _fst_host
-        except ImportError as e:
-            raise LibraryMissing(f"{e}: build it with `python -m flash_spacetime_amd.build`") from e
-        _fst_host.bind_library(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in (
-            "fst_supported", "fst_forward_workspace_bytes", "fst_forward", "fst_backward_workspace_bytes",
-            "fst_backward", "fst_last_error")))
-        _HOST = _fst_host
-    return _HOST
+        _HOST = _load_host()
+    return _HOST or None
 
 
 def last_error() -> str:

@@ -27,11 +27,14 @@ def _same_layout(a: Tensor, b: Tensor) -> bool:
 def _native_backward(dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, scale, out=None):
     """The backward through the host extension: (dq, dk, dv, dw, db), or for an
     interleaved q (k and v None) (dqkv, None, None, dw, db); None where the call is
-    not in the form it takes or runs another than the static plan, for
-    `_run_backward` to run or reject."""
+    not in the form it takes, runs another than the static plan, or the extension
+    is not usable, for `_run_backward` to run or reject."""
     if not (q.is_cuda and tune.static_only()):
         return None
-    return _lib.host().backward(dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, scale, out, _raw_stream(q))
+    host = _lib.host()
+    if host is None:
+        return None
+    return host.backward(dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, scale, out, _raw_stream(q))
 
 
 def _run_backward(dims, q, k, v, pos4, w32, b32, lens, lse, grad_out, scale, vec_shape,

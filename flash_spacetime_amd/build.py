@@ -1,5 +1,5 @@
 """Build the gfx950 HIP library `libflash_spacetime.so` and the host extension
-`_fst_host.so` in the package directory.
+`_fst_host` (its file carries Python's ABI tag) in the package directory.
 
 Every kernel instance family is its own translation unit so hipcc runs them
 in parallel; the objects are linked into one shared library whose C ABI is
@@ -14,14 +14,16 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 BUILD = CSRC / "_build"
+HEADER = PKG.parent / "include" / "flash_spacetime.h"
 LIB = PKG / "libflash_spacetime.so"
-HOST_LIB = PKG / "_fst_host.so"
+HOST_LIB = PKG / f"_fst_host{sysconfig.get_config_var('EXT_SUFFIX')}"
 
 ARCH = os.environ.get("FST_OFFLOAD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
@@ -48,12 +50,13 @@ ROWS_SCHED = ["-mllvm", "--amdgpu-sched-strategy=max-ilp"]
 
 
 def source_hash() -> str:
-    """First 12 hex digits of the SHA-256 of every kernel source: the build id
-    fst_version reports (the tuner's plan cache keys on it)."""
+    """First 12 hex digits of the SHA-256 of every source and the C header: the
+    build id fst_version reports (the tuner's plan cache keys on it, and the
+    host extension is used only with the library of its own build)."""
     import hashlib
 
     h = hashlib.sha256()
-    for p in sorted(CSRC.glob("*.h")) + sorted(CSRC.glob("*.hip")):
+    for p in [p for ext in ("h", "hip", "cpp") for p in sorted(CSRC.glob(f"*.{ext}"))] + [HEADER]:
         h.update(p.name.encode())
         h.update(p.read_bytes())
     return h.hexdigest()[:12]
@@ -76,15 +79,15 @@ def _units():
 
 def _build_host():
     """Compile csrc/fst_host.cpp, the operators' host path (a Python extension
-    against torch's C++ API; no device code)."""
-    import sysconfig
-
+    against torch's C++ API; no device code). It records the build id and the
+    torch it was compiled for, which _lib.host compares."""
     import torch
     from torch.utils import cpp_extension
 
     tmp = HOST_LIB.with_suffix(".so.tmp")
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
-           "-DTORCH_EXTENSION_NAME=_fst_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}"]
+           "-DTORCH_EXTENSION_NAME=_fst_host", f'-DFST_BUILD_ID="{source_hash()}"',
+           f'-DFST_TORCH_VERSION="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}"]
     for inc in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"]):
         cmd += ["-isystem", str(inc)]
     cmd += [str(CSRC / "fst_host.cpp"), "-o", str(tmp)]
@@ -93,6 +96,7 @@ def _build_host():
     if res.returncode != 0:
         raise RuntimeError("host extension failed:\n" + res.stdout + res.stderr)
     os.replace(tmp, HOST_LIB)
+    (PKG / "_fst_host.so").unlink(missing_ok=True)  # the untagged file of earlier builds
 
 
 RESOURCES = BUILD / "kernel_resources.json"

@@ -270,7 +270,11 @@ py::object backward(const Dims& dims, const Tensor& q, const std::optional<Tenso
 
 }  // namespace
 
+// build_id: the library this extension belongs to; torch_version: the torch it
+// was compiled for (compared before bind_library gives it addresses).
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.attr("build_id") = FST_BUILD_ID;
+  m.attr("torch_version") = FST_TORCH_VERSION;
   m.def("bind_library", &bind_library);
   m.def("forward", &forward);
   m.def("backward", &backward);

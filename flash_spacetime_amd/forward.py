@@ -262,9 +262,10 @@ _PLAIN = (Tensor, torch.nn.Parameter)
 def _native_forward(q, k, v, feats, weight, bias, lens, scale, use_attn_bias, use_activation_bias, packed,
                     interleaved=False):
     """The forward through the host extension, or None where the call is not in
-    the form it takes (csrc/fst_host.cpp) or a plan other than the static one
-    is asked for; the Python path below then runs or rejects it. interleaved: q
-    is one contiguous interleaved tensor, k and v are None. Returns (out, lse, q, k, v, pos4,
+    the form it takes (csrc/fst_host.cpp), a plan other than the static one is
+    asked for, or the extension is not usable; the Python path below then runs
+    or rejects it. interleaved: q is one contiguous interleaved tensor, k and v
+    are None. Returns (out, lse, q, k, v, pos4,
     weight, bias, lens, dims, scale) as `_Prepared` and `_run_forward` form them."""
     if not (q.is_cuda and tune.static_only() and (scale is None or type(scale) in (float, int))
             and (k is None) == interleaved and (v is None) == interleaved):
@@ -275,8 +276,11 @@ def _native_forward(q, k, v, feats, weight, bias, lens, scale, use_attn_bias, us
             return None
     if bias is not None and type(bias) not in _PLAIN:
         return None
-    return _lib.host().forward(q, k, v, feats, weight, bias, lens, scale, bool(use_attn_bias),
-                               bool(use_activation_bias), packed, _raw_stream(q))
+    host = _lib.host()
+    if host is None:
+        return None
+    return host.forward(q, k, v, feats, weight, bias, lens, scale, bool(use_attn_bias), bool(use_activation_bias),
+                        packed, _raw_stream(q))
 
 
 def _raw_stream(t: Tensor) -> int:

@@ -273,11 +273,11 @@ void fst_frequencies(int C, float* out);
 const char* fst_last_error(void);
 
 /* Library version string, "flash-spacetime-gfx950 <major>.<minor>.<patch>
- * abi <n> build <id>", id a hash of the kernel sources. The abi number changes with every change of an entry point's
- * arguments or of what a caller must provide (workspace sizes are always
- * queried, so a larger workspace is not an ABI change): abi 2 added the
- * forward's output to fst_backward / fst_backward_phases (the argument
- * `out`, before `scale`). */
+ * abi <n> build <id>", id a hash of the sources. The abi number changes with
+ * every change of an entry point's arguments or of what a caller must provide
+ * (workspace sizes are always queried, so a larger workspace is not an ABI
+ * change): abi 2 added the forward's output to fst_backward /
+ * fst_backward_phases (the argument `out`, before `scale`). */
 const char* fst_version(void);
 
 #ifdef __cplusplus

@@ -10,14 +10,14 @@ step runs hipcc. FST_OFFLOAD_ARCH (default gfx950) and HIPCC are honoured.
 import importlib.util
 from pathlib import Path
 
-from setuptools import setup
+from setuptools import Distribution, setup
 from setuptools.command.build_py import build_py
 
 ROOT = Path(__file__).resolve().parent
 
 
 class BuildWithKernels(build_py):
-    """Compile libflash_spacetime.so and _fst_host.so before the package files are copied."""
+    """Compile libflash_spacetime.so and _fst_host before the package files are copied."""
 
     def run(self):
         spec = importlib.util.spec_from_file_location("fst_build", ROOT / "flash_spacetime_amd" / "build.py")
@@ -25,6 +25,15 @@ class BuildWithKernels(build_py):
         spec.loader.exec_module(mod)
         mod.build()
         super().run()
+
+
+class BinaryDistribution(Distribution):
+    """The wheel holds compiled code: its name carries the Python and platform
+    tags (the host extension also needs the torch it was compiled for, which it
+    records; under another one the operators run without it)."""
+
+    def has_ext_modules(self):
+        return True
 
 
 setup(
@@ -38,7 +47,8 @@ setup(
     install_requires=["torch>=2.4"],
     extras_require={"dev": ["pytest>=7"]},
     packages=["flash_spacetime_amd"],
-    package_data={"flash_spacetime_amd": ["libflash_spacetime.so", "_fst_host.so"]},
+    package_data={"flash_spacetime_amd": ["libflash_spacetime.so", "_fst_host.*.so"]},
+    distclass=BinaryDistribution,
     cmdclass={"build_py": BuildWithKernels},
     zip_safe=False,
 )

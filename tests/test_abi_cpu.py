@@ -8,6 +8,9 @@ device, and report errors the way the reference's operators do.
 
 import ctypes
 import re
+import sys
+import types
+import warnings
 from pathlib import Path
 
 import pytest
@@ -51,6 +54,40 @@ def test_library_exports_every_declared_symbol():
     m = re.fullmatch(r"flash-spacetime-gfx950 \d+\.\d+\.\d+ abi (\d+) build ([0-9a-f]{12})", version)
     assert m and m.group(1) == "2", version
     assert m.group(2) == source_hash(), "the library was built from other sources than these"
+
+
+@needs_lib
+def test_host_extension_belongs_to_the_library():
+    from flash_spacetime_amd import _fst_host
+
+    assert _fst_host.build_id == source_hash(), "the host extension was built from other sources than these"
+    assert _fst_host.torch_version == torch.__version__
+    assert _lib.host() is _fst_host
+
+
+@needs_lib
+@pytest.mark.parametrize("what", ["build_id", "torch_version", "missing"])
+def test_foreign_host_extension_is_not_bound(monkeypatch, what):
+    """One of another build of the library or for another torch is given no
+    addresses; the operators are told to run without it, with one warning."""
+    bound = []
+    fake = types.SimpleNamespace(build_id=source_hash(), torch_version=torch.__version__,
+                                 bind_library=lambda *a: bound.append(a))
+    monkeypatch.setattr(_lib, "_HOST", None)
+    monkeypatch.setattr(flash_spacetime_amd, "_fst_host", fake, raising=False)
+    assert _lib.host() is fake and len(bound) == 1
+    if what == "missing":
+        monkeypatch.delattr(flash_spacetime_amd, "_fst_host")
+        monkeypatch.setitem(sys.modules, "flash_spacetime_amd._fst_host", None)
+    else:
+        setattr(fake, what, "0")
+    monkeypatch.setattr(_lib, "_HOST", None)
+    with pytest.warns(RuntimeWarning, match="host extension"):
+        assert _lib.host() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.host() is None
+    assert len(bound) == 1
 
 
 @needs_lib

@@ -153,6 +153,13 @@ def test_the_usual_forms_take_the_native_path(monkeypatch):
         assert calls and not any(calls)
 
 
+def test_operators_run_without_the_extension(monkeypatch):
+    want = {form: _run(form) for form in ("plain", "packed", "qkv")}
+    monkeypatch.setattr(_lib, "_HOST", False)  # as _lib.host leaves it for an unusable extension
+    for form, res in want.items():
+        assert all(torch.equal(a, e) for a, e in zip(_run(form), res)), form
+
+
 def test_refused_calls_stay_refused():
     q, k, v = (_draw(B, 4, L, D, seed=i) for i in range(3))
     feats, w, b = _draw(B, L, 5, dtype=torch.float32), _draw(D, C, dtype=torch.float32), None
