@@ -1143,10 +1143,16 @@ struct BwdPick {
 // D=32 C=16 in float32 one pass took 7.06 against 9.72 ms), two where it
 // would spill heavily (cfg4, D = C = 64, four waves: 82.8 against 41.2 ms).
 // Eight waves halve the state: at cfg4 one pass (51 registers spilled)
-// took 22.7 ms against 31.7 for two.
+// took 22.7 ms against 31.7 for two. Eight waves of 12 heads (an uneven
+// split) take the passes of four: their smaller state would let one pass do at
+// seven widths, up to 17 % of a step faster (B = 32, L = 768, D = 16, C = 64:
+// 2.42 against 2.90 ms), but its dq is further from 64 bits than that of two in
+// every draw of events of 3000 tokens (by 2 % without a bias, 0.07 % with the
+// activation bias alone).
 template <int HP, int D, int C, int NW>
 constexpr int rows_static_passes() {
-  return HeadSplit<HP, NW>::HW * D + (16 / NW) * C <= 256 ? 1 : 2;
+  constexpr int W = HeadSplit<HP, NW>::EVEN ? NW : 4;
+  return (HP / W) * D + (16 / W) * C <= 256 ? 1 : 2;
 }
 
 template <typename T, int HP, int D, int C, int NW, int NS>
@@ -1209,8 +1215,9 @@ int bwd_launch_t(const BwdParams& prm, int which, hipStream_t stream, int grid, 
   } else {
     int nw = plan_nw(prm.flags, bit_index(FST_PLAN_BWD_T16), bit_index(FST_PLAN_BWD_W8));
     // Two shapes of 12 heads where the eight-wave kernel spills and four waves
-    // are no slower (B = 24, L = 768: D = 64, C = 48 rows 2.21 against 2.31 ms;
-    // D = 64, C = 16 cols 1.34 against 1.32, B = 32 1.69 against 1.74).
+    // are no slower (B = 24, L = 768: D = 64, C = 48 rows 2.21 against 2.31 ms
+    // in one pass; D = 64, C = 16 cols 1.34 against 1.32, B = 32 1.69 against
+    // 1.74).
     if (nw == 0 && HP == 12 && D == 64 && C == (which == 0 ? 48 : 16)) nw = 4;
     const int ns = plan_ns(prm.flags, bit_index(FST_PLAN_BWD_KC16));
     const int split = which == 0 ? pick_split<PR::template F>(nw, ns, 1) : pick_split<PC::template F>(nw, ns, 1);

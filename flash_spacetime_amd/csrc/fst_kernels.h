@@ -693,7 +693,8 @@ constexpr int bit_index(int b) { return b <= 1 ? 0 : 1 + bit_index(b >> 1); }
 // waves kept the float32 kernels at one wave per SIMD (311 to 411 registers a
 // lane at D = 32, C = 16); over eight they run two: H = 12, D = 32, C = 16, B = 32,
 // L = 768, lengths U{16..768}: forward 0.457 -> 0.414 ms, rows 0.795 -> 0.638,
-// cols 1.004 -> 0.683; the other widths -14 to -41 % (rows), -23 to -32 % (cols).
+// cols 1.004 -> 0.683; every width forward -13 to -30 %, rows -9 to -32 %, cols
+// -24 to -34 % (but those two that keep four waves, bwd_launch_t).
 template <int HP, int NW>
 struct HeadSplit {
   static constexpr int HW = (HP + NW - 1) / NW, NBIG = HP - NW * (HW - 1);

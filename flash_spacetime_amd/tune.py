@@ -22,12 +22,14 @@ by 3 % or more (timings vary by a few per cent from run to run), else the
 static choice.
 
 The occupancy, wave, K/V-staging and tile-height variants leave out, lse,
-dq, dk, dv and rowsum unchanged bit for bit (dW and db change only in the
-order their fp32 partial sums are added); the key-chunk and pass variants
-agree with the static choice to rounding. A shape is keyed by the GPU architecture, the
-library version, kind, dtype, H, D, C, the layout and bias flags, and the
-bit lengths of its batch and length (padded) or token count (packed), so the
-ragged batches of one training run share a choice.
+dq, dk, dv and rowsum unchanged bit for bit at the same key chunk and passes
+(dW and db change only in the order their fp32 partial sums are added); the
+key-chunk and pass variants agree with the static choice to rounding. A
+float32 plan with no key-chunk or pass bit takes those its tile height
+prefers, which need not be the static choice's. A shape is keyed by the GPU
+architecture, the library version, kind, dtype, H, D, C, the layout and bias
+flags, and the bit lengths of its batch and length (padded) or token count
+(packed), so the ragged batches of one training run share a choice.
 
 The reference's Triton kernels take fixed tile constants
 (src/flash_spacetime/_tiles.py) and are not autotuned (README.md:86-95); its

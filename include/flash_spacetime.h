@@ -72,12 +72,16 @@ enum fst_flags {
                               takes three separate tensors, forward.py:481). */
   /* Plan bits: a choice among compiled variants of the kernels, for callers
    * that time them. Each group below is one knob of one kernel; at most one
-   * bit of a group may be set, and a group left empty takes the library's
-   * static choice. fst_plans() lists the bits compiled for a shape and
+   * bit of a group may be set, and with none in any group of a kernel it runs
+   * the library's static choice. A group left empty beside others takes the
+   * first variant that fits them in its kernel's order of preference (float32:
+   * 32-key forward chunks first, 16-key (row) backward chunks first, and the
+   * passes that suit the waves), which need not be that of the static choice:
+   * set every group to compare variants. fst_plans() lists the bits compiled for a shape and
    * fst_plan_supported() whether one combination of them is.
    * Variants of the occupancy, wave, K/V-staging and tile-height groups
-   * compute every output row with the same arithmetic: out, lse, dq, dk, dv
-   * and rowsum are the same bit for bit, and dweight / dbias differ only in
+   * compute every output row with the same arithmetic at the same key chunk
+   * and passes: out, lse, dq, dk, dv and rowsum are the same bit for bit, and dweight / dbias differ only in
    * the order in which their fp32 partial sums are added. The key-chunk
    * groups move the points where the online softmax rescales and the order
    * of the sums over keys, and the pass group forms D online or in a first
@@ -169,8 +173,8 @@ int fst_supported(int dtype, int H, int D, int C);
 int fst_plans(int dtype, int H, int D, int C);
 
 /* 1 if the combination `plan` of FST_PLAN_* bits (at most one per group;
- * the empty groups take the static choice) is compiled for (dtype, H, D, C)
- * in both the forward and the backward, else 0.
+ * the empty groups as above) is compiled for (dtype, H, D, C) in both the
+ * forward and the backward, else 0.
  * No reference counterpart (see the plan bits above). */
 int fst_plan_supported(int dtype, int H, int D, int C, int plan);
 

@@ -6,7 +6,9 @@ four-wave tiles that the tile-height plan bits name, at the same key chunk:
 out, lse, dq, dk, dv must agree bit for bit, dW and db to the rounding of
 their partial sums, and all with the float64 oracle at the float32 tolerance
 of the parity tests. Head counts leave padded heads on either kind of wave;
-lengths sit at the edges of tiles and chunks.
+lengths sit at the edges of tiles and chunks. The passes over the keys are
+those of four waves, so the four-wave plan of the backward, with no pass bit,
+gives the static choice's bits at every width.
 """
 
 import pytest
@@ -21,35 +23,32 @@ if torch.cuda.is_available():
     from flash_spacetime_amd import _lib, tune
     from tests.test_plans_gpu import F32, TOL, _inputs, _oracle, _run, _same
 
-# (heads, dim, channels, lengths, packed, bias flags)
+# (heads, dim, channels, lengths, packed, bias flags, keys per forward chunk and
+# passes of the rows kernel in the static choice)
 SHAPES = [
-    (12, 32, 16, [33, 16, 1], False, (True, True)),
-    (12, 32, 32, [31, 64], True, (True, True)),      # 32-key forward chunks
-    (9, 16, 16, [17, 15], False, (True, False)),     # three padded heads
-    (11, 48, 48, [32, 18], True, (True, True)),
-    (10, 16, 64, [47, 2], False, (False, True)),
-    (12, 64, 16, [20, 33], True, (True, True)),      # four-wave cols kernel
-    (12, 64, 48, [35, 1], False, (True, True)),      # four-wave rows kernel
-    (12, 64, 32, [16, 49], False, (False, False)),
+    (12, 32, 16, [33, 16, 1], False, (True, True), 16, 1),
+    (12, 32, 32, [31, 64], True, (True, True), 32, 1),
+    (9, 16, 16, [17, 15], False, (True, False), 16, 1),     # three padded heads
+    (11, 48, 48, [32, 18], True, (True, True), 32, 2),
+    (10, 16, 64, [47, 2], False, (False, True), 16, 2),     # no room for 32 keys
+    (12, 64, 16, [20, 33], True, (True, True), 16, 1),      # four-wave cols kernel
+    (12, 64, 48, [35, 1], False, (True, True), 32, 2),      # four-wave rows kernel
+    (12, 64, 32, [16, 49], False, (False, False), 32, 2),
 ]
 
 
 @pytest.mark.parametrize("case", range(len(SHAPES)))
 def test_uneven_split_matches_four_waves_and_the_oracle(case):
-    heads, dim, chans, lens, packed, flags = SHAPES[case]
+    heads, dim, chans, lens, packed, flags, keys, passes = SHAPES[case]
     print(f"H={heads} D={dim} C={chans} lens={lens} packed={packed} flags={flags}", flush=True)
     args = _inputs(F32, heads, dim, chans, lens, packed, 400 + case)
     tune.set_autotune(False)
     got = _run(args, flags)
-    fkc = _lib.FST_PLAN_FWD_KC16 if chans == 16 else _lib.FST_PLAN_FWD_KC32
-    four = None
-    for kc in (fkc, _lib.FST_PLAN_FWD_KC16):  # 16 keys where the static choice has no room for 32
-        for passes in (_lib.FST_PLAN_BWD_PASS1, _lib.FST_PLAN_BWD_PASS2):
-            plan = (kc | _lib.FST_PLAN_FWD_T16 | _lib.FST_PLAN_BWD_T16 | _lib.FST_PLAN_BWD_KC16 | passes)
-            if tune.plan_supported(F32, heads, dim, chans, plan):
-                with tune.fixed_plan(plan):
-                    four = four or _same(got, _run(args, flags))
-    assert four, "no four-wave plan gives the same bits"
+    plan = (_lib.FST_PLAN_FWD_T16 | (_lib.FST_PLAN_FWD_KC16 if keys == 16 else _lib.FST_PLAN_FWD_KC32)
+            | _lib.FST_PLAN_BWD_T16 | _lib.FST_PLAN_BWD_KC16
+            | (_lib.FST_PLAN_BWD_PASS1 if passes == 1 else _lib.FST_PLAN_BWD_PASS2))
+    with tune.fixed_plan(plan):
+        assert _same(got, _run(args, flags))
     ref = _oracle(args, flags, packed)
     out = got[0]
     if not packed:
@@ -59,3 +58,14 @@ def test_uneven_split_matches_four_waves_and_the_oracle(case):
             continue
         err = rel_err(a, e)
         assert err <= TOL[F32], f"{name} relative error {err:.3e}"
+
+
+@pytest.mark.parametrize("dim, chans", [(16, 64), (32, 16), (32, 48), (32, 64), (48, 16), (48, 32), (48, 48), (48, 64),
+                                        (64, 32)])
+def test_four_wave_backward_without_a_pass_bit_gives_the_same_bits(dim, chans):
+    print(f"D={dim} C={chans}", flush=True)
+    args, flags = _inputs(F32, 12, dim, chans, [130, 57], True, 500 + dim + chans), (True, True)
+    tune.set_autotune(False)
+    got = _run(args, flags)
+    with tune.fixed_plan(_lib.FST_PLAN_BWD_T16):
+        assert _same(got, _run(args, flags))
