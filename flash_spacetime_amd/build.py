@@ -74,6 +74,8 @@ def _units():
                 units.append((f"bwd_{name}", CSRC / "fst_bwd_inst.hip", defs + ["-DFST_BWD_PART=2"]))
             else:
                 units.append((f"bwd_{name}", CSRC / "fst_bwd_inst.hip", defs))
+    # The slowest units first, so that none is left running alone at the end.
+    units.sort(key=lambda u: not u[0].startswith("bwd_f32"))
     return [u for u in units if u[1].exists()]
 
 

@@ -733,7 +733,13 @@ struct BwdColsCfg {
       LDS_BYTES <= 160 * 1024 && HS::OK && RWS >= 1 && EL::OK && (C / 2 / EL::SPLIT) % 4 == 0;
 };
 
-template <typename T, int HP, int D, int C, int NW, int NS>
+// RED: the launch's first workgroups sum dW / db (reduce_block). The tiles'
+// kernel without that code is an instance of its own: beside it 28 of the 236
+// float32 instances spilled more or held a register too many for a wave per
+// SIMD, and calls of any size paid for it (B = 64, L = 768, lengths U{16..768},
+// H = 12, D = 48: C = 16 cols 2.18 -> 2.25 ms, C = 32 2.46 -> 2.52; D = C = 32 at
+// H = 16, D = 64, C = 16 and D = 32, C = 16 at H = 12 0.3 to 0.6 %).
+template <typename T, int HP, int D, int C, int NW, int NS, bool RED>
 __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_cols_kernel(BwdParams prm) {
   using Cfg = BwdColsCfg<T, HP, D, C, NW, NS>;
   constexpr int NT = Cfg::THREADS;
@@ -746,14 +752,18 @@ __global__ __launch_bounds__(64 * (NW > 4 ? NW : 4), 1) void bwd_cols_kernel(Bwd
   const int wave = tid >> 6, lane = tid & 63, g = lane >> 4, n = lane & 15;
   const int tile = wave / NW, ws = wave % NW;
 
-  if ((int)blockIdx.x < prm.red_blocks) {
-    reduce_block<D * C, D>(prm, tid, reinterpret_cast<float*>(smem));
-    return;
+  int wg = blockIdx.x;
+  if constexpr (RED) {
+    if (wg < prm.red_blocks) {
+      reduce_block<D * C, D>(prm, tid, reinterpret_cast<float*>(smem));
+      return;
+    }
+    wg -= prm.red_blocks;
   }
   EventSpec ev = prm.ev;
   ev.blkcum = prm.blkcum_cols;
   EventBlock eb;
-  if (!locate_block(ev, Cfg::KEYS, blockIdx.x - prm.red_blocks, eb)) return;
+  if (!locate_block(ev, Cfg::KEYS, wg, eb)) return;
   const int len = eb.len;
   const int H = prm.H;
   const bool attn = prm.flags & FST_ATTN_BIAS;
@@ -1181,7 +1191,8 @@ int bwd_launch_v(const BwdParams& prm, int which, hipStream_t stream, int grid, 
   } else {
     *rows = K::KEYS;
     if (query) return FST_OK;
-    auto kern = bwd_cols_kernel<T, HP, D, C, NW, NS>;
+    auto kern = prm.red_blocks > 0 ? bwd_cols_kernel<T, HP, D, C, NW, NS, true>
+                                   : bwd_cols_kernel<T, HP, D, C, NW, NS, false>;
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, K::LDS_BYTES) !=
         hipSuccess)
       return FST_ELAUNCH;
