@@ -150,6 +150,8 @@ def kernel_times(inp, seqlens, iters=10, cu=None, plan=0, flags=(True, True), wi
              P(do), P(out) if with_out else None, prep.scale, P(dq), P(dk), P(dv), P(dw), P(db), None, P(bwork),
              bws, sh)
     _lib.check(lib.fst_forward_phases(_lib.FST_PHASE_FWD, *dims, *fargs), "fwd")
+    # The phases timed below read the work list.
+    _lib.check(lib.fst_backward_phases(_lib.FST_PHASE_WORKLIST, *dims, *bargs), "bwd worklist")
     _lib.check(lib.fst_backward_phases(_lib.FST_BWD_ALL, *dims, *bargs), "bwd")
     torch.cuda.synchronize(dev)
     res = {}

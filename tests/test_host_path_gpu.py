@@ -56,7 +56,6 @@ FORMS = {
     "head_groups": {"heads": 17},
     "expanded_grad": {"grad": "expanded"},
     "token_major_grad": {"grad": "token_major"},
-    "float32_grad": {"grad": "float32"},
     "packed": {"layout": "packed"},
     "packed_strided": {"layout": "packed_strided"},
     "packed_int64": {"layout": "packed", "lens": torch.int64},
@@ -111,8 +110,6 @@ def _run(form):
         g = _draw(D, dtype=dt, seed=9).expand(out.shape)
     elif o["grad"] == "token_major":
         g = _draw(B, L, h, D, dtype=dt, seed=9).transpose(1, 2)
-    elif o["grad"] == "float32":
-        g = g.float().to(out.dtype)
     grads = torch.autograd.grad(out, leaves, g, allow_unused=True)
     res = [out.detach(), *grads]
     if lay == "dense":
@@ -135,6 +132,30 @@ def test_native_path_equals_the_python_path(form, monkeypatch):
         if a is not None:
             assert a.dtype == e.dtype and a.shape == e.shape and a.stride() == e.stride(), i
             assert torch.equal(a, e), i
+
+
+@pytest.mark.parametrize("layout", ["dense", "token_major", "packed"])
+def test_gradient_of_another_dtype(layout):
+    """A float32 upstream gradient of bf16 operands (autograd casts it before it
+    gets here) is converted, and the forward's output handed on, as the Python
+    path does."""
+    lead = (sum(LENS), 4) if layout == "packed" else (B, 4, L)
+    q, k, v = (_draw(*lead, D, seed=i) for i in range(3))
+    g = _draw(*lead, D, dtype=torch.float32, seed=9)
+    if layout == "token_major":
+        q, k, v = (_draw(B, L, 4, D, seed=i).transpose(1, 2) for i in range(3))
+    lens = torch.tensor([0, 37, 53, 54] if layout == "packed" else LENS, device=DEV)
+    feats = _draw(*((sum(LENS),) if layout == "packed" else (B, L)), 5, dtype=torch.float32)
+    w, b = _draw(D, C, dtype=torch.float32) / 4, _draw(D, dtype=torch.float32) * 0.02
+    out, lse, qc, kc, vc, pos4, w32, b32, len32, dims, scale = forward._native_forward(
+        q, k, v, feats, w, b, lens, None, True, True, layout == "packed")
+    args = (dims, qc, kc, vc, pos4, w32, b32, len32, lse, g, scale)
+    got = backward._native_backward(*args, out)
+    want = backward._run_backward(*args, forward.vec_shape(dims), out=out)
+    same = backward._native_backward(*args[:9], g.bfloat16(), scale, out)
+    for a, e, s in zip(got, want, same):
+        assert a.dtype == e.dtype and a.stride() == e.stride()
+        assert torch.equal(a, e) and torch.equal(a, s)
 
 
 def test_the_usual_forms_take_the_native_path(monkeypatch):
