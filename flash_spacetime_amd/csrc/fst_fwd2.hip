@@ -587,6 +587,15 @@ struct Fwd2Pick {
                             : D >= 48 && rows_wave_load(HP, D, C) >= 336 ? (Fwd2Cfg<HP, D, C, KC, 2, 8>::FITS ? 2 : 0)
                             : D == 32 && C == 16                         ? (Fwd2Cfg<HP, D, C, KC, 4, 8>::FITS ? 4 : 0)
                                                                          : 0;
+  // Without the bias on the logits the four-wave lane state is smaller and, up
+  // to C = 48, two of its workgroups share a CU at little cost: there eight
+  // waves run only where every tile has a CU to itself (a grid of up to 256
+  // workgroups). Events of 768 tokens, activation bias only, eight against four
+  // waves at 240 / 288 / 1536 tiles: D = 64, C = 48 0.73 / 1.24 / 1.25, C = 32 0.77 /
+  // 1.29 / 1.26, D = C = 48 0.97 / 1.05 / 1.09; no bias 0.78 / 1.11 / 1.11, 0.78 /
+  // 1.13 / 1.12, 0.99 / 1.00 / 1.01 (B = 48, L = 768, heads first: 1.15). With
+  // the logits' bias alone eight waves win throughout (0.45 to 0.81).
+  static constexpr int W8_MAX_GRID_NO_ATTN = C <= 48 && W8 == 2 ? 256 : 0x7fffffff;
   // Occupancy and key-chunk variants a caller may choose instead (the plan
   // bits of include/flash_spacetime.h); the occupancy variants compute every
   // row with the same arithmetic.
@@ -631,7 +640,8 @@ int fwd2_launch_t(const FwdParams& prm, hipStream_t stream, int grid, bool query
     const bool kc32 = prm.flags & FST_PLAN_FWD_KC32;
     const int occ = (prm.flags & FST_PLAN_FWD_OCC2) ? 2 : (prm.flags & FST_PLAN_FWD_OCC3) ? 3 : (kc32 ? 2 : P::OCC);
     if constexpr (P::W8 != 0)
-      if (!(prm.flags & (FST_PLAN_FWD_OCC2 | FST_PLAN_FWD_OCC3)) && !kc32)
+      if (!(prm.flags & (FST_PLAN_FWD_OCC2 | FST_PLAN_FWD_OCC3)) && !kc32 &&
+          ((prm.flags & FST_ATTN_BIAS) || grid <= P::W8_MAX_GRID_NO_ATTN))
         return fwd2_launch_occ<HP, D, C, 16, P::W8, 8>(prm, stream, grid, query);
     if (kc32) return occ == 2 ? fwd2_launch_occ<HP, D, C, 32, 2>(prm, stream, grid, query) : FST_EUNSUPPORTED;
     if (occ == 3) return fwd2_launch_occ<HP, D, C, 16, 3>(prm, stream, grid, query);

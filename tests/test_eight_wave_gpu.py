@@ -1,7 +1,9 @@
 """GPU tests of the bf16 forward's and cols kernel's eight-wave instances.
 
 Where the library's static choice runs eight waves (heavy lane states at 16
-padded heads, wide heads at 8, and the cols kernel's 12 heads padded to 16),
+padded heads, wide heads at 8, and the cols kernel's 12 heads padded to 16;
+without the bias on the logits the forward only in grids of up to 256
+workgroups),
 every row and key is computed with the arithmetic of the four-wave instances
 that the occupancy plan bits name: out, lse, dq, dk, dv must agree bit for
 bit, dW and db to the rounding of their float32 partial sums, and all with
@@ -32,6 +34,9 @@ SHAPES = [
     (9, 48, 64, [20, 1], True, (True, True)),
     (8, 64, 16, [33, 15], True, (True, True)),      # cols kernel, four waves per SIMD
     (5, 48, 32, [17, 48], False, (False, False)),
+    (13, 48, 48, [33, 15], False, (False, True)),   # forward: few tiles, eight waves
+    (16, 64, 32, [17, 1] * 100, True, (False, True)),  # more than 256 workgroups, four waves
+    (14, 64, 48, [9] * 260, False, (False, False)),
 ]
 
 
