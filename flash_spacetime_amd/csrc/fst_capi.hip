@@ -51,12 +51,17 @@ static int rows_head_padding(int dtype, int flags, int H, int D, int C) {
 // the four-wave instance spills at 12 (D = 48, C >= 48) and the eight-wave one
 // at 16 does not (H = 12, D = 48, B = 48, L = 768, lengths U{16..768}: C = 64
 // 0.515 -> 0.359 ms, C = 48 0.367 -> 0.327; at D = 64 the four extra heads cost
-// more than the spills, C = 64 0.397 -> 0.454). Its plan bits name the
-// four-wave variants, at head_padding.
+// more than the spills, C = 64 0.397 -> 0.454). With one bias or none the
+// four-wave instance holds its state and 12 heads are a quarter to a half
+// faster (one bias: B = 48, L = 768, C = 48 0.341 at 16 against 0.242 ms, C = 64 0.339
+// against 0.291; 72 packed events of up to 768 tokens 0.873 / 0.609 and 0.858 /
+// 0.649; no bias 0.235 / 0.151, 0.658 / 0.518). Its plan bits name the four-wave
+// variants, at head_padding.
 static int cols_head_padding(int dtype, int flags, int H, int D, int C) {
   const int hp = head_padding(H);
   if (dtype != FST_BF16 || (flags & (FST_PLAN_COLS_OCC2 | FST_PLAN_COLS_OCC3))) return hp;
-  return hp == 12 && D == 48 && C >= 48 ? 16 : hp;
+  const bool both = (flags & FST_ATTN_BIAS) && (flags & FST_ACT_BIAS);
+  return hp == 12 && D == 48 && C >= 48 && both ? 16 : hp;
 }
 
 // fp32 frequency ladder exp(-i * ln(1e4) / (C/2)) evaluated with the same

@@ -34,6 +34,7 @@ SHAPES = [
     (9, 48, 64, [20, 1], True, (True, True)),
     (8, 64, 16, [33, 15], True, (True, True)),      # cols kernel, four waves per SIMD
     (5, 48, 32, [17, 48], False, (False, False)),
+    (11, 48, 64, [18, 33], True, (True, False)),    # cols kernel, one bias: 12 heads on four waves
     (13, 48, 48, [33, 15], False, (False, True)),   # forward: few tiles, eight waves
     (16, 64, 32, [17, 1] * 100, True, (False, True)),  # more than 256 workgroups, four waves
     (14, 64, 48, [9] * 260, False, (False, False)),
