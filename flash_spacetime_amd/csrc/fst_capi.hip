@@ -33,7 +33,11 @@ static int head_padding(int H) { return H <= 4 ? 4 : (H <= 8 ? 8 : (H <= 12 ? 12
 // the four-wave instance would spill, so that it runs eight waves (padded
 // heads compute on a real head's data and store nothing; 12 heads split over
 // eight waves unpadded). The scratch between the rows and cols kernel is laid
-// out by H, so each pads as it likes.
+// out by H, so each pads as it likes. At D = 48, C = 64 with a bias the unpadded
+// split loses where a token's heads are adjacent (72 packed events of up to 768
+// tokens: both biases 1.156 against 1.122 ms padded to 16, activation bias 1.001
+// against 0.954; an event of 1500 tokens 0.403 / 0.386, 0.367 / 0.342) and wins
+// heads first (B = 48, L = 768 0.626 / 0.646).
 // The eight-wave, one-workgroup plan (FST_PLAN_ROWS_W8) pads to a multiple of
 // 8; the four-wave plan and the eight-wave, two-workgroup plan (which gives
 // waves 4 to 7 one head fewer where 8 does not divide the padding) keep
@@ -44,6 +48,8 @@ static int rows_head_padding(int dtype, int flags, int H, int D, int C) {
   if (flags & FST_PLAN_ROWS_W8) return (hp + 7) & ~7;
   if (flags & (FST_PLAN_ROWS_W4 | FST_PLAN_ROWS_W8X2)) return hp;
   if (hp == 4 && rows_wave_load(hp, D, C) >= 160) return 8;
+  const bool token_rows = flags & (FST_PACKED | FST_TOKEN_MAJOR), bias = flags & (FST_ATTN_BIAS | FST_ACT_BIAS);
+  if (hp == 12 && D == 48 && C == 64 && token_rows && bias) return 16;
   return hp;
 }
 

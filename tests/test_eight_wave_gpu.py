@@ -60,3 +60,16 @@ def test_eight_waves_match_four_and_the_oracle(case):
             continue
         err = rel_err(a, e)
         assert err <= TOL[BF], f"{name} relative error {err:.3e}"
+
+
+@pytest.mark.parametrize("packed", [True, False], ids=["packed", "heads_first"])
+@pytest.mark.parametrize("flags", [(True, True), (False, True), (False, False)])
+def test_rows_of_twelve_heads_padded_or_split_unevenly(packed, flags):
+    """D = 48, C = 64: the rows kernel pads to 16 heads where a token's heads are
+    adjacent and a bias is on, else splits 12 unevenly: the bits of the plan
+    that names the padded one either way."""
+    args = _inputs(BF, 10, 48, 64, [35, 16, 1], packed, 350)
+    tune.set_autotune(False)
+    got = _run(args, flags, True)
+    with tune.fixed_plan(_lib.FST_PLAN_ROWS_W8):
+        assert _same(got, _run(args, flags, True))
