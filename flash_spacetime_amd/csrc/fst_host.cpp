@@ -3,8 +3,8 @@
 // operands in the form nearly every call gives them. What the Python layer
 // (forward.py, backward.py) decides by some forty tensor calls and a 25-argument
 // ctypes call is decided here in one: 63 -> 42 us a forward of one 187-token
-// event (its kernel takes 17), 252 -> 154 us a forward and backward of 64 events
-// of up to 192 tokens (its kernels take 120).
+// event (its kernel takes 16), 252 -> 154 us a forward and backward of 64 events
+// of up to 192 tokens (its kernels then took 138, now 119).
 //
 // Both functions return None for anything but that form (unsupported shapes
 // and dtypes, mixed devices, tensor subclasses, lengths that are not integers
